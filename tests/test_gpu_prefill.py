@@ -57,6 +57,33 @@ def test_batch_equals_per_token_gemv(torch_dev, N, K, M):
         np.testing.assert_array_equal(yb[m].cpu().numpy(), yo)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (5, 64, 64), (31, 320, 130), (64, 320, 1030),          # 64 x 32 tiles, four K groups
+    (600, 1088, 200), (97, 8256, 64), (545, 1920, 320),    # 128 x 32, two K groups
+    (1999, 1088, 130), (1030, 2112, 70), (260, 13824, 64),  # 128 x 64
+    (3400, 1344, 70), (1285, 3840, 2500), (500, 13824, 190)])  # 256 x 128
+def test_batch_shapes_against_whole_sums(torch_dev, M, N, K):
+    """Every shape that the plan picks, with ragged tokens, rows that end inside a
+    tile and odd and even counts of 64-column chunks, against the whole-number sums
+    in float64 (exact: |sum| < 2^53) and the one fp32 product of each."""
+    from tenzo_amd import ops
+    torch = torch_dev
+    print(f"tl1_batch shapes M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+    w = torch.randint(-1, 2, (N, K), dtype=torch.int8, device="cuda", generator=g)
+    u = (w + 1).to(torch.uint8).reshape(N // 64, 2, 32, K // 2, 2)
+    nib = u[..., 0] | (u[..., 1] << 2)
+    packed = (nib[:, 0] | (nib[:, 1] << 4)).transpose(1, 2).contiguous().reshape(-1)
+    wp = ops.tl1_repack(packed, N, K)
+    codes, q, _ = ops.rmsnorm_quant31(torch.randn((M, K), device="cuda", generator=g))
+    yb, ab = ops.bitlinear_tl1_batch(codes, q, wp, 0.0173, N, K, want_acc=True)
+    acc = codes[:, :K].double() @ w.double().T
+    assert torch.equal(ab.double(), acc)
+    scale = ops.actq_inv_scale(q) * torch.tensor(0.0173, device="cuda")
+    assert torch.equal(yb, acc.float() * scale[:, None])
+
+
 @pytest.mark.parametrize("tile", [142, 242, 442, 222, 422, 221, 421, 412, 411, 811])
 def test_batch_every_tile_shape(torch_dev, tile):
     """Every workgroup tile shape gives the same exact sums, with a ragged
