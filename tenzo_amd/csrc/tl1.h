@@ -53,5 +53,12 @@ int tl1_pick_splits(int64_t nb, int64_t KS, int64_t M);
 int launch_tl1_mfma(const int8_t* codes, const tenzo_hip_actq_t* q, const void* w_packed,
                     const RowScales& rs, int64_t M, int64_t N, int64_t K, float* y,
                     const float* resid, int32_t* acc_out, hipStream_t st, int tile);
+// gate | up of M tokens in one product whose rows leave as act = max(0, gate)^2 * up
+// ([M][F]; :1616-1620): launch_tl1_mfma's rows and actquant mode 3's arithmetic on them.
+// Weights: F gate rows, then F up rows; F % 64 == 0 and the sizes that _fits accepts.
+bool tl1_mfma_glu_fits(int64_t M, int64_t F, int64_t K);
+int launch_tl1_mfma_glu(const int8_t* codes, const tenzo_hip_actq_t* q, const void* w_packed,
+                        float gate_scale, float up_scale, int64_t M, int64_t F, int64_t K,
+                        float* act, hipStream_t st);
 
 }  // namespace tz

@@ -688,6 +688,41 @@ int launch_tl1_mfma(const int8_t* codes, const tenzo_hip_actq_t* q, const void* 
     return TENZO_ERROR_INVALID_ARGUMENT;
 }
 
+bool tl1_mfma_glu_fits(int64_t M, int64_t F, int64_t K) {
+    const int64_t KS = ceil_div(K, 64);
+    // (32-bit offsets over the whole weight matrix and over 128 rows of outputs)
+    return F % 64 == 0 && 2 * F <= (1 << 22) && M * KS * 64 <= (int64_t)INT32_MAX &&
+           K <= (1 << 20) && F / 32 * KS * 1024 < (int64_t)UINT32_MAX;
+}
+
+int launch_tl1_mfma_glu(const int8_t* codes, const tenzo_hip_actq_t* q, const void* w_packed,
+                        float gate_scale, float up_scale, int64_t M, int64_t F, int64_t K,
+                        float* act, hipStream_t st) {
+    const int64_t N = 2 * F, nb = N / 64, KS = ceil_div(K, 64);
+    RowScales rs{};
+    rs.n = 2;
+    rs.end[0] = F;
+    rs.end[1] = INT64_MAX;
+    rs.scale[0] = gate_scale;
+    rs.scale[1] = up_scale;
+    // Shapes as for the plain product, two row tiles to a wave (one of each matrix).
+    // us at 13824 x 2560 (128x32 / 128x64 with two K groups / 128x64 / 256x128): 20 tokens
+    // 6.5 8.0 8.9 16.3; 128 tokens 9.3 8.8 9.5 16.5; 256 17.3 16.0 13.1 18.2; 512 29.2
+    // 30.9 23.8 20.8; 2048 113 121 84.8 65.6 (the plain product: 71.1 and a row twice as
+    // long for the quantizer to read).
+    if (ceil_div(nb, 2) * ceil_div(M, 32) <= 256)
+        return launch_wide<2, 1, 2, 2, 1, 4, true>(codes, q, w_packed, rs, M, N, KS, act, nullptr,
+                                                   nullptr, st);
+    if (ceil_div(nb, 2) * ceil_div(M, 64) <= 256)
+        return launch_wide<2, 2, 2, 2, 1, 4, true>(codes, q, w_packed, rs, M, N, KS, act, nullptr,
+                                                   nullptr, st);
+    if (ceil_div(nb, 4) * ceil_div(M, 128) < 160)
+        return launch_wide<2, 2, 1, 2, 1, 4, true>(codes, q, w_packed, rs, M, N, KS, act, nullptr,
+                                                   nullptr, st);
+    return launch_wide<4, 2, 1, 2, 2, 3, true>(codes, q, w_packed, rs, M, N, KS, act, nullptr,
+                                               nullptr, st);
+}
+
 }  // namespace tz
 
 using namespace tz;

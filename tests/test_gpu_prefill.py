@@ -171,8 +171,52 @@ def test_engine_prefill_equals_token_by_token(torch_dev, ctx, n):
             np.testing.assert_array_equal(a.logits(), b.logits())
 
 
+@pytest.mark.parametrize("n,F", [(20, 6912), (100, 6912), (140, 6912), (600, 4160)])
+def test_engine_prefill_gate_up_shapes(torch_dev, n, F):
+    """The gate | up product with the activation in its epilogue, in each of its
+    shapes (20: 128 x 32 tiles, 100: 128 x 64 with two K groups, 140: 128 x 64,
+    600: 256 x 128, whose last tile is half empty at 65 row blocks): bit for bit
+    the per-token path's gate, up and activation."""
+    from tenzo_amd import engine as eng_mod, synth
+    cfg = synth.DecodeConfig(hidden=512, n_q_heads=4, n_kv_heads=1, n_layers=1, ffn=F,
+                             vocab=512, max_seq=640, theta=10000.0)
+    sm = synth.make_model(cfg, seed=n, ctx=0)
+    toks = np.random.default_rng(n).integers(0, cfg.vocab, n).astype(np.int32)
+    print(f"engine prefill gate|up n={n} F={F}", flush=True)
+    a, b = _engine_pair(eng_mod, cfg, sm)
+    with a, b:
+        rows = []
+        for t in toks:
+            a.prefill(int(t))
+            rows.append(a.buffer("x"))
+        b.prefill_batch(toks, exact=True)
+        np.testing.assert_array_equal(rows[-1], b.buffer("x"))
+        for i in (n // 3, n // 2):  # other tokens' rows, as the last of a shorter prompt
+            b.reset()
+            b.prefill_batch(toks[:i], exact=True)
+            np.testing.assert_array_equal(rows[i - 1], b.buffer("x"))
+
+
+def test_engine_prefill_passes(torch_dev):
+    """2100 tokens in two passes (2048 + 52 rows) equal the same tokens as two
+    prompts of 300 (small buffers) and 1800 rows (buffers grown)."""
+    from tenzo_amd import engine as eng_mod, synth
+    cfg = synth.DecodeConfig(hidden=512, n_q_heads=4, n_kv_heads=1, n_layers=2, ffn=512,
+                             vocab=1024, max_seq=2200, theta=10000.0)
+    sm = synth.make_model(cfg, seed=72, ctx=0)
+    toks = np.random.default_rng(4).integers(0, cfg.vocab, 2100).astype(np.int32)
+    a, b = _engine_pair(eng_mod, cfg, sm)
+    with a, b:
+        a.prefill_batch(toks, exact=True)
+        b.prefill_batch(toks[:300], exact=True)
+        b.prefill_batch(toks[300:], exact=True)
+        for x, y in zip(a.get_kv(2100), b.get_kv(2100)):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_array_equal(a.buffer("x"), b.buffer("x"))
+
+
 def test_engine_prefill_longer_than_one_pass(torch_dev):
-    """600 tokens: two passes of the 512-row buffers, attention over up to 19
+    """600 tokens: more than the small buffers' 512 rows, attention over up to 19
     chunks per query, G = 4 query heads per kv head."""
     from tenzo_amd import engine as eng_mod, synth
     cfg = synth.DecodeConfig(hidden=512, n_q_heads=4, n_kv_heads=1, n_layers=2, ffn=512,
