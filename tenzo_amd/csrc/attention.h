@@ -96,8 +96,8 @@ int launch_attn_paged(const AttnPagedLaunch& L, hipStream_t st);
 // 0 .. pos0+i. exact: with the chunking and arithmetic of a decode step at
 // that position (chunk by chunk, then the decode merge), so every output
 // equals the one n sequential decode steps produce bit for bit; otherwise a
-// streaming pass per query (one wave, 64-token blocks, online softmax), equal
-// to within fp32 rounding of the softmax sums and far faster. q / k_new /
+// streaming pass over the prefix for 16 or 64 rows at a time (online softmax),
+// equal to within fp32 rounding of the softmax sums and far faster. q / k_new /
 // v_new are rows of row_stride elements (q at column 0, k and v where the
 // pointers say); out rows are out_stride apart.
 struct AttnPrefill {

@@ -1267,6 +1267,386 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(AttnArgs a) {
     }
 }
 
+// Prefill attention, streaming form, for longer prefixes: a workgroup takes 64 rows
+// (64 / G consecutive queries x the G heads of one kv head), 32 to a wave, and KG pairs of
+// waves share a row half's key tiles of 32 tokens (group k: tiles k, k + KG, ...). Each
+// round of KG tiles is laid out in LDS once for the waves of both halves (the 16-row kernel
+// above loads and converts every code once per 16 rows, and keeps the row statistics in
+// 16-lane butterflies). A round is bound by the vector unit: ~380 instructions a wave
+// beside 28 MFMAs.
+//
+// Scores, S^T = K Q^T on v_mfma_i32_32x32x32_i8: the cache codes are the operand as they
+// are, and a query row enters as a 24-bit fixed-point number of its largest |q| in three
+// signed byte digits, so the sums are whole numbers and exact (fp16 hi + lo parts carry 22
+// bits and need the codes converted). Lane l = 32g + n holds row n's scores of tokens
+// 8a + 4g + b in register 4a + b: a row's maximum and sum are one lane's registers and one
+// exchange with lane l ^ 32, and its weights are already the second operand of
+// O^T = V^T W^T if k slot (g, 4a' + b) of step s means token 16s + 8a' + 4g + b.
+// Values on v_mfma_f32_32x32x16_f16: weights as power-of-two scaled fp16 hi + lo parts (a
+// scale per tile), a tile's products in an accumulator of their own, added to the row's in
+// fp32 (left in the MFMA's accumulator over a prefix, the sums drift: it does not round to
+// nearest).
+//
+// LDS, a tile: K token t's 16-byte piece p at place p ^ (t / 2 % 8) of its 128 bytes; V^T
+// dim d at row d ^ (d / 16 % 4) (the low two bits), its piece (s, g) at place
+// (2s + g) ^ (d / 4 % 4) of 64 bytes. The 16 lanes that a read serves together touch the
+// 64 banks once each, and a write's 32 lanes twice.
+constexpr int kFlashRows = 64;
+constexpr int kFlashTile = 4096 + 8192;  // K codes, V^T in fp16
+
+typedef _Float16 h8a __attribute__((ext_vector_type(8)));
+typedef float f16a __attribute__((ext_vector_type(16)));
+typedef int i16a __attribute__((ext_vector_type(16)));
+typedef int i4a __attribute__((ext_vector_type(4)));
+
+// The three signed byte digits of four fixed-point numbers |w| <= 0x7f7f7f, most significant
+// first: byte i of digit j is number i's.
+__device__ __forceinline__ void digits4(const int (&w)[4], int (&dig)[3]) {
+    uint32_t t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = (uint32_t)w[i] + 0x808080u;  // bytes: digit + 128
+    const uint32_t a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);  // bytes 0, 0, 1, 1
+    const uint32_t a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+    const uint32_t c01 = __builtin_amdgcn_perm(t[1], t[0], 0x06020602u);  // byte 2 of both
+    const uint32_t c23 = __builtin_amdgcn_perm(t[3], t[2], 0x06020602u);
+    dig[2] = (int)(__builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u);
+    dig[1] = (int)(__builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x80808080u);
+    dig[0] = (int)(__builtin_amdgcn_perm(c23, c01, 0x05040100u) ^ 0x80808080u);
+}
+
+template <int G, int KG>
+__global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArgs a) {
+    constexpr int NT = 128 * KG;        // threads
+    constexpr int QP = kFlashRows / G;  // queries per workgroup
+    constexpr int kQS = kD + 4;         // padded row of the rotated queries
+    constexpr int kMerge = KG * 16384;  // half of the key groups' sums
+    constexpr int kBuf = kMerge > kFlashRows * kQS * 4 ? kMerge : kFlashRows * kQS * 4;
+    __shared__ __align__(16) char buf[kBuf];                 // queries; KG tiles; merge
+    __shared__ __align__(16) float ksl[KG][32], vsl[KG][32];  // the tiles' scales
+    __shared__ float ml[2][2][KG][32];
+    __shared__ float vdn[KG];  // 2^-e of the tile's V scales (below)
+    static_assert(kBuf >= KG * kFlashTile, "a tile per key group");
+    const int h = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave & 1, kg = wave >> 1;  // row half, key group
+    const int n = lane & 31, g = lane >> 5;
+    const int qb = (gridDim.y - 1 - blockIdx.y) * QP;  // (the longest prefixes first)
+    const int nq = min(QP, a.pos_n - qb);
+    const int nkey = a.pos + qb + nq;  // keys 0 .. the last live query
+    const int ntile = (nkey + 31) / 32;
+    const int64_t cache_head = (int64_t)h * a.max_seq;
+    const __amdgpu_buffer_rsrc_t rk = att_rsrc(a.kc + cache_head * kD, (uint32_t)nkey * kD);
+    const __amdgpu_buffer_rsrc_t rv = att_rsrc(a.vc + cache_head * kD, (uint32_t)nkey * kD);
+    const uint16_t* ksb = a.ks + cache_head;
+    const uint16_t* vsb = a.vs + cache_head;
+
+    // one thread's share of a round of KG tiles (tokens past the last read zero codes): of
+    // two tiles K's piece ti % 8 of token ti / 8 and V's 4 x 4 block of tokens 4 (ti / 32) ..
+    // and dims 4 (ti % 32) .., ti = tid % 256; one scale (the first 32 KG threads K's, then V's)
+    const int ti = tid & 255, tx = tid >> 8;
+    uint4 kr[2];
+    uint32_t vr[2][4];
+    uint16_t sr;
+    auto load = [&](int round) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const uint32_t t0 = (uint32_t)(KG * round + 2 * tx + x) * 32 * kD;
+            kr[x] = __builtin_bit_cast(
+                uint4, __builtin_amdgcn_raw_buffer_load_b128(rk, t0 + (uint32_t)ti * 16, 0, 0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                vr[x][e] = __builtin_amdgcn_raw_buffer_load_b32(
+                    rv, t0 + (uint32_t)(4 * (ti >> 5) + e) * kD + 4 * (ti & 31), 0, 0);
+        }
+        const int t = min(KG * 32 * round + tid % (32 * KG), nkey - 1);
+        sr = (tid & (32 * KG) ? vsb : ksb)[t];
+    };
+    load(0);
+
+    // ---- RoPE on the rows (:460-481); rows of dead queries are zero. All loads first ----
+    float* qs = reinterpret_cast<float*>(buf);
+    {
+        constexpr int kIt = kFlashRows * 16 / NT;  // four pairs at a time
+        float4 x0[kIt], x1[kIt], cs[kIt], sn[kIt];
+#pragma unroll
+        for (int r = 0; r < kIt; ++r) {
+            const int i = tid + NT * r, m = i >> 4, j = 4 * (i & 15);
+            const int b = qb + min(m / G, nq - 1);
+            const float* rope = a.rope + (int64_t)(a.pos + b) * kD + j;
+            const float* qv = a.q + (int64_t)b * a.q_stride + (int64_t)(h * G + m % G) * kD + j;
+            x0[r] = *reinterpret_cast<const float4*>(qv);
+            x1[r] = *reinterpret_cast<const float4*>(qv + 64);
+            cs[r] = *reinterpret_cast<const float4*>(rope);
+            sn[r] = *reinterpret_cast<const float4*>(rope + 64);
+        }
+#pragma unroll
+        for (int r = 0; r < kIt; ++r) {
+            const int i = tid + NT * r, m = i >> 4, j = 4 * (i & 15);
+            const bool live = m / G < nq;
+            const float p[4] = {x0[r].x, x0[r].y, x0[r].z, x0[r].w};
+            const float q[4] = {x1[r].x, x1[r].y, x1[r].z, x1[r].w};
+            const float c[4] = {cs[r].x, cs[r].y, cs[r].z, cs[r].w};
+            const float z[4] = {sn[r].x, sn[r].y, sn[r].z, sn[r].w};
+            float lo[4], hi[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lo[e] = live ? __builtin_fmaf(p[e], c[e], -__fmul_rn(q[e], z[e])) : 0.0f;
+                hi[e] = live ? __builtin_fmaf(p[e], z[e], __fmul_rn(q[e], c[e])) : 0.0f;
+            }
+            *reinterpret_cast<float4*>(qs + m * kQS + j) = make_float4(lo[0], lo[1], lo[2], lo[3]);
+            *reinterpret_cast<float4*>(qs + m * kQS + j + 64) =
+                make_float4(hi[0], hi[1], hi[2], hi[3]);
+        }
+    }
+    __syncthreads();
+
+    // the rows' digits: step s, dims 32 s + 16 g ..; the largest |q| scaled to [2^22, 2^23),
+    // or half of that where it would pass the digits' range
+    i4a qd[4][3];
+    float c2, qin;  // (qin: a score's unit; c2: the same times log2(e))
+    {
+        const float* qrow = qs + (rg * 32 + n) * kQS + 16 * g;
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mx = fmaxf(mx, fabsf(qrow[32 * s + e]));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        int sh = fp16_span_exp(mx) + 9;
+        if (ldexpf(mx, sh) > 8355711.0f) --sh;
+        const float up = ldexpf(1.0f, sh);
+        qin = ldexpf(1.0f, -sh);
+        c2 = 1.44269502f * qin;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                int w[4], dig[3];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = (int)rintf(qrow[32 * s + 4 * e + i] * up);
+                digits4(w, dig);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) qd[s][j][e] = dig[j];
+            }
+    }
+    const int qi = (rg * 32 + n) / G;
+    const int prow = qi < nq ? a.pos + qb + qi : -1;  // the row's position (-1: dead, all masked)
+    const int pmin = a.pos + qb + min(rg * 32 / G, nq - 1);  // the wave's first row's
+
+    float mr = -1e30f, lr = 0.0f;  // (the scores' maximum in units of qin)
+    f16a o[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[dt] = f16a{};
+    const char* kt = buf + kg * kFlashTile;
+    const char* vt = kt + 4096;
+    const uint32_t koff = (uint32_t)n * 128u, kswz = (uint32_t)((g ^ (n >> 1 & 7)) * 16);
+    const uint32_t voff = (uint32_t)((n & 28) | ((n ^ (n >> 4)) & 3)) * 64u;
+    const uint32_t vswz = (uint32_t)((g ^ (n >> 2 & 3)) * 16);
+
+    auto step = [&](int t0, bool masked) {
+        i16a d0{}, d1{}, d2{};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const i4a k = *reinterpret_cast<const i4a*>(kt + koff + (kswz ^ (uint32_t)(2 * s * 16)));
+            d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][0], d0, 0, 0, 0);
+            d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][1], d1, 0, 0, 0);
+            d2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][2], d2, 0, 0, 0);
+        }
+        f16a d;
+        float mx = -1e30f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 f = *reinterpret_cast<const float4*>(&ksl[kg][8 * q + 4 * g]);
+            const float fs[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = 4 * q + e;
+                const float dot = __builtin_fmaf((float)d0[j], 65536.0f,
+                                                 (float)((d1[j] << 8) + d2[j]));
+                d[j] = __fmul_rn(dot, fs[e]);
+            }
+        }
+        if (masked) {  // (uniform: the tiles on the diagonal and past it)
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (t0 + 8 * (j >> 2) + 4 * g + (j & 3) > prow) d[j] = -1e30f;
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, d[j]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // weights e^(qin (s - m)) as 2^(c2 s - c2 m): one rounding of the exponent, no more
+        // than the scores' own
+        const float mn = fmaxf(mr, mx), mc = mn * c2;
+        const float rs = mr > -1e30f ? __builtin_amdgcn_exp2f((mr - mn) * c2) : 0.0f;  // (1 if mr stays)
+        mr = mn;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) d[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(d[j], c2, -mc));
+        if (masked) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (t0 + 8 * (j >> 2) + 4 * g + (j & 3) > prow) d[j] = 0.0f;
+        }
+        float ls = 0.0f;
+        h8a wh[2], wl[2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 f = *reinterpret_cast<const float4*>(&vsl[kg][8 * q + 4 * g]);
+            const float fs[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ls += d[4 * q + e];
+                float w = __fmul_rn(d[4 * q + e], fs[e]);  // (fs: s_v 2^e)
+                // (opaque: fused with the product, one of hi's two uses would round once
+                // instead of twice, and lo would not be its remainder on a tie)
+                asm("" : "+v"(w));
+                const _Float16 hi = (_Float16)w;
+                wh[q >> 1][4 * (q & 1) + e] = hi;
+                wl[q >> 1][4 * (q & 1) + e] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, w);
+            }
+        }
+        lr = __builtin_fmaf(lr, rs, ls);
+        const float dn = vdn[kg];
+        if (__any(rs != 1.0f)) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) o[dt][j] *= rs;
+        }
+#pragma unroll
+        for (int dp = 0; dp < 4; dp += 2) {
+            f16a t[2] = {f16a{}, f16a{}};
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                h8a v[2];
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    v[x] = *reinterpret_cast<const h8a*>(vt + (dp + x) * 2048 +
+                                                         (voff ^ (uint32_t)(x * 128)) +
+                                                         (vswz ^ (uint32_t)(2 * s * 16)));
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    t[x] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[x], wh[s], t[x], 0, 0, 0);
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    t[x] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[x], wl[s], t[x], 0, 0, 0);
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    o[dp + x][j] = __builtin_fmaf(t[x][j], dn, o[dp + x][j]);
+        }
+    };
+
+    uint32_t e64 = 0x64006400u;  // (a VGPR operand of v_perm_b32)
+    asm volatile("" : "+v"(e64));
+    const h2a bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const uint32_t kw = (uint32_t)((ti >> 3) * 128 + ((ti & 7) ^ (ti >> 4 & 7)) * 16);
+    // V: dims 4 c + f (c = ti % 32) of tokens 4 Q .. (Q = ti / 32): 8 bytes of piece (s, g)
+    const int vQ = ti >> 5, vc = ti & 31;
+    const uint32_t vw = (uint32_t)(vc * 256 + ((2 * (vQ >> 2) + (vQ & 1)) ^ (vc & 3)) * 16 +
+                                   (vQ >> 1 & 1) * 8);
+    const int nround = (ntile + KG - 1) / KG;
+    for (int round = 0; round < nround; ++round) {
+        __syncthreads();  // the queries (first), or the tiles before, are read
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            char* tk = buf + (2 * tx + x) * kFlashTile;
+            *reinterpret_cast<uint4*>(tk + kw) = kr[x];
+            uint32_t v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = vr[x][e] ^ 0x80808080u;
+            const uint32_t t01a = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u);
+            const uint32_t t01b = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u);
+            const uint32_t t23a = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u);
+            const uint32_t t23b = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const uint32_t sel = (f & 1) ? 0x07030502u : 0x07010500u;
+                const h2a p01 =
+                    __builtin_bit_cast(h2a, __builtin_amdgcn_perm(e64, f < 2 ? t01a : t01b, sel)) + bias;
+                const h2a p23 =
+                    __builtin_bit_cast(h2a, __builtin_amdgcn_perm(e64, f < 2 ? t23a : t23b, sel)) + bias;
+                *reinterpret_cast<h4a*>(tk + 4096 + vw + ((f ^ (vc >> 2)) & 3) * 64) =
+                    h4a{p01.x, p01.y, p23.x, p23.y};
+            }
+        }
+        if (tid < 64 * KG) {
+            const float f = half_bits_to_float(sr);
+            if (tid < 32 * KG) ksl[tid >> 5][tid & 31] = __fmul_rn(f, kScaleFactor);
+            else {
+                // the tile's power-of-two scale of W = p * s_v, from its largest s_v
+                float mx = row16_max(f);
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                const int sh = fp16_span_exp(mx);
+                vsl[(tid >> 5) - KG][tid & 31] = ldexpf(f, sh);
+                if ((tid & 31) == 0) vdn[(tid >> 5) - KG] = ldexpf(1.0f, -sh);
+            }
+        }
+        __syncthreads();
+        if (round + 1 < nround) load(round + 1);
+        const int t0 = (KG * round + kg) * 32;
+        if (t0 < nkey) step(t0, t0 + 31 > pmin);
+    }
+
+    // the key groups' sums join group 0's, half of them at a time
+    const float lt = lr + __shfl_xor(lr, 32, 64);
+    if (g == 0) {
+        ml[0][rg][kg][n] = mr;
+        ml[1][rg][kg][n] = lt;
+    }
+    __syncthreads();
+    float M = -1e30f, L = 0.0f, e = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) M = fmaxf(M, ml[0][rg][k][n]);
+#pragma unroll
+    for (int k = 0; k < KG; ++k) {
+        const float m = ml[0][rg][k][n];
+        const float w = m > -1e30f ? expf((m - M) * qin) : 0.0f;
+        L = __builtin_fmaf(w, ml[1][rg][k][n], L);
+        e = k == kg ? w : e;
+    }
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[dt][j] *= e;
+#pragma unroll
+    for (int half = KG / 2; half >= 1; half /= 2) {
+        // [dim][row] of groups half .. 2 half - 1
+        float* om = reinterpret_cast<float*>(buf) + (kg % half * 2 + rg) * 32 * kD;
+        if (kg >= half && kg < 2 * half) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    om[(32 * dt + 8 * (j >> 2) + 4 * g + (j & 3)) * 32 + n] = o[dt][j];
+        }
+        __syncthreads();
+        if (kg < half) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    o[dt][j] += om[(32 * dt + 8 * (j >> 2) + 4 * g + (j & 3)) * 32 + n];
+        }
+        __syncthreads();
+    }
+    if (kg > 0 || prow < 0) return;
+    float* out = a.out + (int64_t)(qb + qi) * a.out_stride +
+                 (int64_t)(h * G + (rg * 32 + n) % G) * kD;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float r[4];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) r[e4] = __fdiv_rn(o[dt][4 * q + e4], L);
+            *reinterpret_cast<float4*>(out + 32 * dt + 8 * q + 4 * g) =
+                make_float4(r[0], r[1], r[2], r[3]);
+        }
+}
+
 // Prefill append: RoPE on k and the INT8 quantization of k and v for the
 // tokens at positions pos .. pos + n - 1, with the arithmetic of the decode
 // kernel's append (so the cache matches one decode step per token). Grid
@@ -1418,6 +1798,24 @@ int launch_attn_prefill(const AttnPrefill& P, hipStream_t st) {
     if (rc) return rc;
     if (!P.exact && (G == 1 || G == 2 || G == 4 || G == 8)) {
         a.pos_n = P.n;
+        // The 64-row kernel from a prefix of 256 keys on (20 / 5 heads, 16-row kernel against
+        // 64-row, with the append, us: 100 tokens 13.5 / 13.8, 256: 21.5 / 17.4, 512: 41.3 /
+        // 23.9, 1500: 144 / 63; 16 tokens after 8000: 304 / 161); four key groups to a
+        // workgroup while one round of them holds the grid (1500: two groups 65.5, four 63.0;
+        // 2048, 640 workgroups: 88.4 / 103). Error against float64, 1500 / 8000 keys:
+        // 3.7e-8 / 5.3e-7 before, 3.2e-8 / 2.9e-7.
+        if (P.pos0 + P.n >= 256) {
+            const dim3 fg((unsigned)P.Hkv, (unsigned)ceil_div(P.n, kFlashRows / G));
+            const bool four = (int64_t)fg.x * fg.y <= 512;
+#define FLASH_CASE(GG)                                                                        \
+    if (G == GG && four)                                                                      \
+        hipLaunchKernelGGL((attn_prefill_flash_kernel<GG, 4>), fg, dim3(512), 0, st, a);      \
+    if (G == GG && !four)                                                                     \
+        hipLaunchKernelGGL((attn_prefill_flash_kernel<GG, 2>), fg, dim3(256), 0, st, a);
+            FLASH_CASE(1) FLASH_CASE(2) FLASH_CASE(4) FLASH_CASE(8)
+#undef FLASH_CASE
+            return launch_status("attn_prefill_flash_kernel");
+        }
         dim3 grid((unsigned)ceil_div(P.n, 16 / G), P.Hkv);
         switch (G) {
             case 1: hipLaunchKernelGGL(attn_prefill_mfma_kernel<1>, grid, dim3(256), 0, st, a); break;

@@ -380,5 +380,37 @@ def test_engine_prefill_streaming_attention(torch_dev, ctx, n, G):
         assert ta == tb
 
 
+@pytest.mark.parametrize("ctx,n,Hq,Hkv", [(200, 60, 4, 4), (0, 256, 4, 2), (250, 77, 4, 1),
+                                          (255, 1, 4, 1), (0, 300, 8, 1), (0, 2100, 16, 4),
+                                          (31, 2200, 16, 16)])
+def test_engine_prefill_streaming_64_rows(torch_dev, ctx, n, Hq, Hkv):
+    """The 64-row streaming attention (prefixes of 256 keys and more; four key groups
+    to a workgroup, two for the last two prompts) against the exact form, for every
+    count of heads per kv head, ragged ends of rows and of key tiles, and rows whose
+    prefix ends inside the first tiles. Each token's second-layer K and V codes come
+    from its own first-layer attention: rounded codes may flip on a tie (a flip moves a
+    few of a row's codes by one), a row with a key too many or too few differs
+    throughout."""
+    from tenzo_amd import engine as eng_mod, synth
+    cfg = synth.DecodeConfig(hidden=128 * Hq, n_q_heads=Hq, n_kv_heads=Hkv, n_layers=2, ffn=512,
+                             vocab=512, max_seq=ctx + n + 8, theta=10000.0)
+    sm = synth.make_model(cfg, seed=n, ctx=ctx)
+    toks = np.random.default_rng(n).integers(0, cfg.vocab, n).astype(np.int32)
+    print(f"streaming 64 rows ctx={ctx} n={n} Hq={Hq} Hkv={Hkv}", flush=True)
+    a, b = _engine_pair(eng_mod, cfg, sm)
+    with a, b:
+        a.prefill_batch(toks, exact=True)
+        b.prefill_batch(toks)
+        ka, va, *_ = a.get_kv(ctx + n)
+        kb, vb, *_ = b.get_kv(ctx + n)
+        for u, v in ((ka, kb), (va, vb)):
+            np.testing.assert_array_equal(u[0], v[0])
+            d = np.abs(u[1].astype(np.int32) - v[1])  # [Hkv][token][128]
+            print("codes that differ", (d > 0).mean(), "largest share of a row",
+                  (d > 0).mean(axis=(0, 2)).max(), flush=True)
+            assert (d > 0).mean() < 0.01
+            assert np.sqrt((d.astype(np.float64) ** 2).mean(axis=(0, 2))).max() < 4.0
+
+
 def rel(a, b):
     return np.abs(np.asarray(a, np.float64) - b).max() / max(np.abs(b).max(), 1e-30)
