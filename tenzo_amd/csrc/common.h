@@ -220,33 +220,42 @@ __device__ __forceinline__ void chain_block(const float4* row, float& s) {
 // one float4 (one wait) at a time. Only lanes 0..7 read: an LDS read then
 // returns 8 x 16 bytes instead of 64 x 16. The n % 8 tail is added to chain
 // 0; the result is returned in every lane of the wave.
+// (chain_run: the whole float4s and single terms of n8 terms a chain, by lanes 0..7;
+// chain_total: the chains' combination.)
+__device__ __forceinline__ void chain_run(const float* row, int n8, float& s) {
+    const float4* r4 = reinterpret_cast<const float4*>(row);
+    const int nq = n8 >> 2;  // whole float4s of a chain
+    int q = 0;
+    for (; q + 16 <= nq; q += 16) chain_block<16>(r4 + q, s);
+    if (q + 8 <= nq) {
+        chain_block<8>(r4 + q, s);
+        q += 8;
+    }
+    if (q + 4 <= nq) {
+        chain_block<4>(r4 + q, s);
+        q += 4;
+    }
+    for (; q < nq; ++q) chain_block<1>(r4 + q, s);
+    for (int k = nq * 4; k < n8; ++k) s = __builtin_fmaf(row[k], row[k], s);
+}
+__device__ __forceinline__ float chain_total(float s) {
+    const float c0 = lane_f(s, 0), c1 = lane_f(s, 1), c2 = lane_f(s, 2), c3 = lane_f(s, 3);
+    const float c4 = lane_f(s, 4), c5 = lane_f(s, 5), c6 = lane_f(s, 6), c7 = lane_f(s, 7);
+    return ((c0 + c4) + (c2 + c6)) + ((c1 + c5) + (c3 + c7));
+}
 __device__ __forceinline__ float chain_sumsq_wave(const float* ct, int ld, int64_t n) {
     const int j = threadIdx.x & 7;
-    const int n8 = (int)(n >> 3), nq = n8 >> 2;  // whole float4s of a chain
+    const int n8 = (int)(n >> 3);
     float s = 0.0f;
     if ((threadIdx.x & 63) < 8) {
-        const float4* row = reinterpret_cast<const float4*>(ct + j * ld);
-        int q = 0;
-        for (; q + 16 <= nq; q += 16) chain_block<16>(row + q, s);
-        if (q + 8 <= nq) {
-            chain_block<8>(row + q, s);
-            q += 8;
-        }
-        if (q + 4 <= nq) {
-            chain_block<4>(row + q, s);
-            q += 4;
-        }
-        for (; q < nq; ++q) chain_block<1>(row + q, s);
-        for (int k = nq * 4; k < n8; ++k) s = __builtin_fmaf(ct[j * ld + k], ct[j * ld + k], s);
+        chain_run(ct + j * ld, n8, s);
         if (j == 0)
             for (int64_t t = (int64_t)n8 * 8; t < n; ++t) {
                 const float v = ct[(int)(t & 7) * ld + n8];
                 s = __builtin_fmaf(v, v, s);
             }
     }
-    const float c0 = lane_f(s, 0), c1 = lane_f(s, 1), c2 = lane_f(s, 2), c3 = lane_f(s, 3);
-    const float c4 = lane_f(s, 4), c5 = lane_f(s, 5), c6 = lane_f(s, 6), c7 = lane_f(s, 7);
-    return ((c0 + c4) + (c2 + c6)) + ((c1 + c5) + (c3 + c7));
+    return chain_total(s);
 }
 
 // Signed 8-bit dot of 4 lanes + accumulator (v_dot4_i32_i8).
