@@ -539,6 +539,264 @@ q4_0_f16_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w,
     if (row < N && sub == 0) y[(int64_t)b * N + row] = acc;
 }
 
+// ------------------------------------------------------------------------
+// Q4_0 / Q8_0 weights times several activation rows on int8 MFMA (up to 8 rows a
+// workgroup; the kernels above read and unpack the weights once per row).
+//
+// y[b][n] = sum over blocks of d_n * sum_j a_bj q_nj. Per block of 32 elements the inner
+// sum is exact: a row's 32 activations become 31-bit fixed-point numbers of the block's
+// largest magnitude (a power-of-two scale s_b), in four signed byte digits, and one
+// v_mfma_i32_32x32x32_i8 multiplies them (first operand, row 8 j + b: digit j of
+// activation row b) by 32 weight rows' codes (second operand, as they are; a Q4_0 nibble
+// as 16 (q - 8)). Lane l = 32 g + n then holds weight row n's sums for activation rows
+// 4 g + e (e < 4) in registers 4 j + e, and adds d_n s_b (the digits' sums) to its fp32
+// sums: 28 vector instructions a block where products of the codes themselves take over
+// 128 for 8 rows. fp32 and fp16 activations of the same values give the same bits.
+//
+// A workgroup owns 32 weight rows; wave v takes blocks 8 v .. 8 v + 7 of each chunk of 8 W
+// blocks, and the waves' sums are added in LDS pairwise. Neighbouring lanes fetch
+// neighbouring 16 bytes of a row's 8 blocks (lanes that read whole blocks, or their own MFMA
+// row, cost the address unit a clock each: 1.5 and 3 times the time), one chunk ahead, and
+// leave them in the wave's LDS as they are; the chunk's digits are made once for all waves,
+// from activations that were fetched a chunk ahead too. What is left is vector work: a third
+// digits (of the same activations in every workgroup), the rest unpacking and the sums.
+// 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 19.9 | 48.1, 16 rows 36 | 113
+// (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 19.8 | 29.3.
+// ------------------------------------------------------------------------
+typedef int gi4 __attribute__((ext_vector_type(4)));
+typedef int gi16 __attribute__((ext_vector_type(16)));
+typedef uint32_t gu4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// four neighbouring activations, as loaded
+template <typename TA>
+struct Act4;
+template <>
+struct Act4<float> {
+    typedef float4 type;
+    static __device__ __forceinline__ float4 value(float4 v) { return v; }
+};
+template <>
+struct Act4<uint16_t> {
+    typedef uint2 type;
+    static __device__ __forceinline__ float4 value(uint2 v) {
+        return make_float4(half_bits_to_float((uint16_t)v.x), half_bits_to_float((uint16_t)(v.x >> 16)),
+                           half_bits_to_float((uint16_t)v.y), half_bits_to_float((uint16_t)(v.y >> 16)));
+    }
+};
+
+// 16-byte unit of digit row n, half g of a block: the rows of a block (reads) and the halves
+// of a row's 8 blocks (writes) both spread over the banks, at constant distances
+constexpr int kGgBlock = 66;
+__device__ __forceinline__ int frag_unit(int blk, int g, int n) {
+    return blk * kGgBlock + g * (kGgBlock / 2) + n;
+}
+
+template <bool Q4, typename TA, int W>  // W waves
+__global__ void __launch_bounds__(64 * W, 8 / W)
+gguf_rows_kernel(const TA* __restrict__ act, const uint8_t* __restrict__ w, float* __restrict__ y,
+                 int K, int N, int B) {
+    constexpr int kBytes = Q4 ? 18 : 34;
+    constexpr int kUnits = kBytes / 2;     // 16-byte units of a row's 8 blocks
+    constexpr int kLoads = (32 * kUnits + 63) / 64;
+    constexpr int kChunk = 8 * W;
+    __shared__ uint4 dig[kChunk * kGgBlock];  // the chunk's digits
+    __shared__ uint4 raw[W][kLoads * 64];  // the waves' weights: [row][kUnits]
+    __shared__ __align__(16) float sa[kChunk][8];
+    __shared__ int odd_chunk;              // the last chunk with an infinity or a NaN
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, g = lane >> 5;
+    const int b0 = blockIdx.y * 8;
+    const int nb = min(8, B - b0);
+    act += (int64_t)b0 * K;
+    const int nbk = K / 32;  // (even)
+    const int row0 = blockIdx.x * 32;
+
+    const uint8_t* rows = w + (int64_t)row0 * nbk * kBytes;
+    const uint32_t row_bytes = (uint32_t)nbk * kBytes;
+    uint32_t wrow[kLoads], wpos[kLoads];  // this lane's units: start of the row, byte in the segment
+    uint4 wq[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int u = lane + 64 * i, r = u / kUnits;
+        wrow[i] = (uint32_t)min(r, min(31, N - 1 - row0)) * row_bytes;
+        wpos[i] = 16 * (uint32_t)(u - r * kUnits);
+    }
+    auto load_codes = [&](int bk) {
+        if (bk + 8 <= nbk) {
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const gu4 v = *reinterpret_cast<const gu4*>(rows + (uint32_t)(wrow[i] + bk * kBytes + wpos[i]));
+                wq[i] = uint4{v[0], v[1], v[2], v[3]};
+            }
+        } else if (bk < nbk) {  // the row's last blocks: word by word, none past its end
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                uint32_t v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    v[k] = *reinterpret_cast<const uint32_t*>(
+                        rows + (uint32_t)(wrow[i] + min(bk * kBytes + wpos[i] + 4 * k, row_bytes - 4)));
+                wq[i] = uint4{v[0], v[1], v[2], v[3]};
+            }
+        }
+    };
+
+    // activations: thread tid takes elements 4 (tid % 8) .. + 3 of the chunk's block tid / 8
+    const int ablk = tid >> 3, l8 = tid & 7;
+    typedef typename Act4<TA>::type Act;
+    Act x[8];
+    auto load_acts = [&](int bk0) {
+        const bool in = bk0 + ablk < nbk;
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+            x[b] = in && b < nb ? *reinterpret_cast<const Act*>(act + (int64_t)b * K +
+                                                                (bk0 + ablk) * 32 + 4 * l8)
+                                : Act{};
+    };
+    auto store_digits = [&](int bk0) {
+        uint32_t* o = reinterpret_cast<uint32_t*>(dig);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            if (b >= nb) break;  // (uniform; idle rows' sums are not stored)
+            const float4 xb = Act4<TA>::value(x[b]);
+            const float v[4] = {xb.x, xb.y, xb.z, xb.w};
+            uint32_t mb = 0;  // the largest |x|, as bits (infinities and NaN on top)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mb = max(mb, __float_as_uint(v[e]) & 0x7fffffffu);
+            mb = max(mb, (uint32_t)dpp_i<kDppXor1>((int)mb));
+            mb = max(mb, (uint32_t)dpp_i<kDppXor2>((int)mb));
+            mb = max(mb, (uint32_t)dpp_i<kDppHalfMirror>((int)mb));
+            // the largest |x| 2^sh in [2^29, 2^30): within the four digits' range
+            const bool fin = mb < 0x7f800000u;
+            const int sh = min(30 - __builtin_amdgcn_frexp_expf(__uint_as_float(mb)), 145);
+            uint32_t t[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                t[e] = (uint32_t)(int)__builtin_amdgcn_ldexpf(v[e], sh) + 0x80808080u;
+            const uint32_t a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);
+            const uint32_t a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+            const uint32_t c01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);
+            const uint32_t c23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+            const uint32_t dg[4] = {__builtin_amdgcn_perm(c23, c01, 0x07060302u),
+                                    __builtin_amdgcn_perm(c23, c01, 0x05040100u),
+                                    __builtin_amdgcn_perm(a23, a01, 0x07060302u),
+                                    __builtin_amdgcn_perm(a23, a01, 0x05040100u)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[4 * frag_unit(ablk, l8 >> 2, 8 * j + b) + (l8 & 3)] = dg[j] ^ 0x80808080u;
+            if (l8 == 0) {
+                sa[ablk][b] = fin ? __builtin_amdgcn_ldexpf(1.0f, -sh - (Q4 ? 4 : 0))
+                                  : __uint_as_float(0x7fc00000u);
+                if (!fin) odd_chunk = bk0;
+            }
+        }
+    };
+
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // activation rows 4 g + e
+    if (tid == 0) odd_chunk = -1;
+    for (int i = tid; i < kChunk * 8; i += 64 * W) sa[i >> 3][i & 7] = 0.0f;
+    load_acts(0);
+    load_codes(8 * wave);
+    __syncthreads();
+    for (int bk0 = 0; bk0 < nbk; bk0 += kChunk) {
+        const int bk = bk0 + 8 * wave;
+        store_digits(bk0);
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) raw[wave][lane + 64 * i] = wq[i];
+        if (bk0 + kChunk < nbk) {
+            load_acts(bk0 + kChunk);
+            load_codes(bk + kChunk);
+        }
+        __syncthreads();
+        const bool slow = odd_chunk == bk0;
+        const int m = min(8, nbk - bk);
+        const uint32_t* wr = reinterpret_cast<const uint32_t*>(&raw[wave][n * kUnits]);
+        // block j's sums and weight scale. Even blocks start on a word with their scale; odd
+        // ones have their codes on words, and the scale before them
+        auto product = [&](int j4, int i, float (&f)[4]) {  // block j4 + i, j4 % 4 == 0
+            const int blk = 8 * wave + j4 + i;
+            const uint4 au = dig[frag_unit(blk, g, n)];
+            const float4 s4 = *reinterpret_cast<const float4*>(&sa[blk][4 * g]);
+            const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
+            const int at = kBytes * j4 / 4 + ((kBytes * i) >> 2), c = at + (i & 1) + (Q4 ? 0 : 4 * g);
+            uint32_t q[4] = {wr[c], wr[c + 1], wr[c + 2], wr[c + 3]};
+            if (!(i & 1)) {
+                const uint32_t x = wr[c + 4];
+                q[0] = __builtin_amdgcn_alignbyte(q[1], q[0], 2);
+                q[1] = __builtin_amdgcn_alignbyte(q[2], q[1], 2);
+                q[2] = __builtin_amdgcn_alignbyte(q[3], q[2], 2);
+                q[3] = __builtin_amdgcn_alignbyte(x, q[3], 2);
+            }
+            if (Q4) {  // elements 0..15 in the low nibbles (g = 0), 16..31 in the high
+#pragma unroll
+                for (int k = 0; k < 4; ++k) q[k] = ((q[k] << (g ? 0 : 4)) & 0xf0f0f0f0u) ^ 0x80808080u;
+            }
+            const gi16 r = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                gi4{(int)au.x, (int)au.y, (int)au.z, (int)au.w},
+                gi4{(int)q[0], (int)q[1], (int)q[2], (int)q[3]}, gi16{}, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                f[e] = sc[e] * __builtin_fmaf((float)((r[e] << 8) + r[4 + e]), 65536.0f,
+                                              (float)((r[8 + e] << 8) + r[12 + e]));
+            return half_bits_to_float((uint16_t)(i & 1 ? wr[at] >> 16 : wr[at] & 0xffffu));
+        };
+        // a chunk's blocks are added pairwise: short chains of fp32 sums (m is even)
+        float sum[4] = {};
+#pragma unroll 1
+        for (int j = 0; j < m; j += 4) {
+            float f[4][4], d[4];
+            d[0] = product(j, 0, f[0]), d[1] = product(j, 1, f[1]);
+            if (j + 4 <= m)
+                d[2] = product(j, 2, f[2]), d[3] = product(j, 3, f[3]);
+            else
+                for (int e = 0; e < 4; ++e) f[2][e] = f[3][e] = d[2] = d[3] = 0.0f;
+            if (slow) {  // (uniform) blocks with an infinity or a NaN: their products one by one
+                const int8_t* wb = reinterpret_cast<const int8_t*>(wr);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int blk = j + (i >> 2), b = 4 * g + (i & 3);
+                    const float sc = sa[8 * wave + blk][b];
+                    if (blk >= m || sc == sc) continue;
+                    float p = 0.0f;
+#pragma unroll 1
+                    for (int k = 0; k < 32; ++k) {
+                        const int8_t* c = wb + kBytes * blk + 2;
+                        const float q = Q4 ? (float)((c[k & 15] >> (k & 16 ? 4 : 0)) & 15) - 8.0f
+                                           : (float)c[k];
+                        p = __builtin_fmaf(to_f32<TA>(act[(int64_t)b * K + (bk + blk) * 32 + k]), q, p);
+                    }
+                    f[i >> 2][i & 3] = p;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sum[e] += __builtin_fmaf(f[1][e], d[1], f[0][e] * d[0]) +
+                          __builtin_fmaf(f[3][e], d[3], f[2][e] * d[2]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += sum[e];
+        __syncthreads();  // the chunk has been read
+    }
+    float* red = reinterpret_cast<float*>(dig);  // [wave][activation row][weight row]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[(wave * 8 + 4 * g + e) * 32 + n] = acc[e];
+    __syncthreads();
+    if (tid < 256) {
+        const int b = tid >> 5;
+        if (row0 + n < N && b < nb) {
+            float v[W];
+#pragma unroll
+            for (int q = 0; q < W; ++q) v[q] = red[(q * 8 + b) * 32 + n];
+#pragma unroll
+            for (int h = W / 2; h; h >>= 1)
+#pragma unroll
+                for (int q = 0; q < h; ++q) v[q] += v[q + h];
+            y[(int64_t)(b0 + b) * N + row0 + n] = v[0];
+        }
+    }
+}
+
 // Q4_0 weights x Q8_0 activations: per block the exact int32 dot
 // sum_j (q_j - 8) qa_j = dot4(q, qa) - 8 * sum_j qa_j, then an fp32 FMA with
 // d_w * d_a. Activations staged in LDS as codes + fp32 scales + code sums.
@@ -1292,9 +1550,36 @@ static int pick_lpr(int ngroups) {
     return l;
 }
 
+// gguf_rows_kernel where it is the faster one. It needs words at every second block
+// (K % 64 == 0) and aligned activations. Its time hardly depends on B, that of the kernels
+// above is B rows' unpacking: us at N x K = 4096 x 4096, here | above, 4 rows 10.8 | 12.4 (Q8_0)
+// and 8.8 | 11.3 (Q4_0, fp32), 2 rows 9.7 | 8.0 and 8.1 | 7.4; fp16 rows times Q4_0 are products
+// of half pairs there: 8 rows 11.0 | 12.3, 4 rows 9.0 | 7.2, and over 8192 weight rows 3 rows
+// 26.1 | 24.9, 4 rows 26.8 | 32.6 (22016 x 4096). Without whole groups of 8 blocks the kernels
+// above take two bytes at a time: 2 rows, 5504 x 3200, 9.4 | 22.7 (Q8_0), 7.8 | 66.8 (Q4_0,
+// fp32), 7.9 | 11.9 (Q4_0, fp16). Eight waves a workgroup while each has a CU to itself
+// (8192 x 4096, 8 rows: 15.1, four waves 19.7), else four, two to a CU (14336: 22.6, eight 27.1).
+template <bool Q4, typename TA>
+static bool launch_gguf_rows(const TA* act, const uint8_t* w, float* y, int K, int N, int B,
+                             hipStream_t st) {
+    if (K % 64 != 0 || ((uintptr_t)w & 3) != 0 || ((uintptr_t)act & 15) != 0) return false;
+    constexpr bool kPairs = Q4 && sizeof(TA) == 2;
+    const bool full = K % 256 == 0 && ((uintptr_t)w & 15) == 0;
+    const int64_t sums = (int64_t)B * N;
+    if (full ? sums < (kPairs ? 32768 : 16384) || B < (kPairs ? 4 : 2) : sums < (kPairs ? 8192 : 4096))
+        return false;
+    const dim3 grid((unsigned)ceil_div(N, 32), (unsigned)ceil_div(B, 8));
+    if ((int64_t)grid.x * grid.y <= 256)
+        hipLaunchKernelGGL((gguf_rows_kernel<Q4, TA, 8>), grid, dim3(512), 0, st, act, w, y, K, N, B);
+    else
+        hipLaunchKernelGGL((gguf_rows_kernel<Q4, TA, 4>), grid, dim3(256), 0, st, act, w, y, K, N, B);
+    return true;
+}
+
 template <typename TA>
 static int launch_q4_0(const TA* act, const uint8_t* w, float* y, int K, int N, int B,
                        hipStream_t st) {
+    if (launch_gguf_rows<true>(act, w, y, K, N, B, st)) return launch_status("gguf_rows_kernel");
     const int nbk = K / 32;
     const int lpr = pick_lpr((nbk + 7) / 8);
     const bool full = K % 256 == 0 && ((uintptr_t)act & 15) == 0 && ((uintptr_t)w & 15) == 0;
@@ -1319,6 +1604,7 @@ static int launch_q4_0(const TA* act, const uint8_t* w, float* y, int K, int N, 
 template <typename TA>
 static int launch_q8_0(const TA* act, const uint8_t* w, float* y, int K, int N, int B,
                        hipStream_t st) {
+    if (launch_gguf_rows<false>(act, w, y, K, N, B, st)) return launch_status("gguf_rows_kernel");
     const int nbk = K / 32;
     const int lpr = pick_lpr((nbk + 7) / 8);
     const bool full = K % 256 == 0 && ((uintptr_t)act & 15) == 0 && ((uintptr_t)w & 15) == 0;
@@ -1482,6 +1768,8 @@ TENZO_HIP_API int tenzo_hip_gemv_q4_0(const void* act, int act_dtype, const uint
     hipStream_t st = (hipStream_t)stream;
     if (act_dtype == 0) return launch_q4_0((const float*)act, w, y, K, N, B, st);
     // fp16 activations: the packed fp16 dot kernel
+    if (launch_gguf_rows<true>((const uint16_t*)act, w, y, K, N, B, st))
+        return launch_status("gguf_rows_kernel");
     const int nbk = K / 32;
     const int lpr = pick_lpr((nbk + 7) / 8);
     const size_t smem = (size_t)K * 2;

@@ -116,6 +116,48 @@ def test_q8_0_weights(torch_dev, N, K, B):
     np.testing.assert_array_equal(y32, y)  # the same fp32 activations either way
 
 
+@pytest.mark.parametrize("N,K,B", [(8191, 64, 2), (5504, 3200, 9), (4097, 2304, 8),
+                                   (8225, 4096, 17), (16400, 448, 4), (2049, 576, 4)])
+@pytest.mark.parametrize("kind", ["q4_0", "q8_0"])
+def test_gguf_several_rows(torch_dev, kind, N, K, B):
+    """Rows enough for the matrix-core kernel: row tiles, chunks and the segments of 8 blocks
+    end partly filled (N % 32, K % 256 and K % 2048 != 0), groups of 8 activation rows too, with
+    four and eight waves. The sums are exact but for their fp32 additions, at most
+    K / 32 + 16 roundings of partial sums of at most sum |a w|. A row whose blocks hold an
+    infinity or a NaN gives what its products give, and leaves the others alone."""
+    from tenzo_amd import ops
+    torch = torch_dev
+    print(f"{kind} N={N} K={K} B={B}", flush=True)
+    rng = np.random.default_rng(N + 7 * K + B)
+    d = (rng.standard_normal((N, K // 32)) * 0.01).astype(np.float16)
+    if kind == "q4_0":
+        q = rng.integers(0, 16, size=(N, K), dtype=np.uint8)
+        w, W = formats.q4_0_pack(q, d), q4_dense(q, d)
+    else:
+        q = rng.integers(-128, 128, size=(N, K)).astype(np.int8)
+        w, W = formats.q8_0_pack(q, d), q.astype(np.float64) * np.repeat(d.astype(np.float64), 32, axis=1)
+    a16 = rng.standard_normal((B, K)).astype(np.float16)
+    a16[:, 32:64] *= np.float16(2.0 ** -12)  # blocks of other magnitudes, one of zeros
+    a16[1, :32] = 0
+    run = getattr(ops, "gemv_" + kind)
+    w = dev(torch, w)
+    y = run(dev(torch, a16.astype(np.float32)), w, K, N).cpu().numpy()
+    a = a16.astype(np.float64)
+    bound = (K / 32 + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(W).T)
+    assert (np.abs(y - a @ W.T) <= bound).all()
+    y16 = run(dev(torch, a16), w, K, N).cpu().numpy()
+    assert (np.abs(y16 - a @ W.T) <= bound).all()
+    bad = a16.copy()
+    bad[0, K - 1] = np.inf
+    bad[1, 3] = np.nan
+    z = run(dev(torch, bad), w, K, N).cpu().numpy()
+    assert np.isnan(z[1]).all()
+    with np.errstate(invalid="ignore"):
+        last = np.float64(np.inf) * W[:, K - 1]  # (NaN where the code is 0)
+    np.testing.assert_array_equal(z[0], last)
+    np.testing.assert_array_equal(z[2:], y16[2:])
+
+
 @pytest.mark.parametrize("N,K", [(64, 32), (11008, 4096), (100, 2304), (257, 8192), (33, 288)])
 def test_q4_0_q8_0_activations(torch_dev, N, K):
     from tenzo_amd import ops
