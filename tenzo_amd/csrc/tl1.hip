@@ -352,14 +352,16 @@ actquant_reg_kernel(const float* __restrict__ x, const float* __restrict__ w, fl
             const float e[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                float r = roundf(__fmul_rn(e[k], scale_act));
-                if (QMAX == 127) r = fminf(fmaxf(r, -128.0f), 127.0f);
-                c[k] = (int)r;
+                if (QMAX == 31) {
+                    c[k] = act_code<31>(e[k], scale_act);
+                } else {  // (a NaN takes the lower bound)
+                    const float r = roundf(__fmul_rn(e[k], scale_act));
+                    c[k] = (int)fminf(fmaxf(r, -128.0f), 127.0f);
+                }
             }
         }
         csum += (c[0] + c[1]) + (c[2] + c[3]);
-        *reinterpret_cast<uint32_t*>(cm + i) = (uint32_t)(c[0] & 0xff) | ((uint32_t)(c[1] & 0xff) << 8) |
-                                              ((uint32_t)(c[2] & 0xff) << 16) | ((uint32_t)(c[3] & 0xff) << 24);
+        *reinterpret_cast<uint32_t*>(cm + i) = pack4(c[0], c[1], c[2], c[3]);
     }
     csum = block256_sum_i32(csum, redi);
     if (t == 0) {
@@ -552,9 +554,8 @@ tl1_gemv_f32_kernel(const uint4* __restrict__ w, const float* __restrict__ x, in
     for (int j = 0; j < J; ++j) {
         int c[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = (int)roundf(__fmul_rn(xv[j][e], scale));
-        cs[t + 256 * j] = (uint32_t)(c[0] & 0xff) | (uint32_t)(c[1] & 0xff) << 8 |
-                          (uint32_t)(c[2] & 0xff) << 16 | (uint32_t)(c[3] & 0xff) << 24;
+        for (int e = 0; e < 4; ++e) c[e] = act_code<31>(xv[j][e], scale);
+        cs[t + 256 * j] = pack4(c[0], c[1], c[2], c[3]);
         csum += (c[0] + c[1]) + (c[2] + c[3]);
     }
     csum = block256_sum_i32(csum, redi);  // (its block barriers publish the codes)
@@ -581,6 +582,141 @@ tl1_gemv_f32_kernel(const uint4* __restrict__ w, const float* __restrict__ x, in
         const float inv_scale = __fmul_rn(amax, 1.0f / 31.0f);
         y[m * N + row] = (float)(tot - csum) * __fmul_rn(inv_scale, rs.scale[j]);
     }
+}
+
+// ------------------------------------------------------------------------
+// The same unit for several rows: a workgroup takes R rows of x and 64 weight rows, and
+// multiplies them with v_mfma_i32_16x16x64_i8. Each of its four waves quantizes R / 4 rows
+// (in its registers, J float4 to a lane, with the arithmetic above) into LDS codes; then wave v
+// takes super-chunk groups v, v + 4, ... of four super-chunks (s .. s + 3) and all four 16-row
+// tiles. Lane l = 16 g + i:
+//   A (weights): row i of the tile in super-chunk s + g (its whole 16-byte record, one load);
+//      step j takes dword j, unpacked,
+//   B (codes):   row i % R of x, the same columns: 16 bytes at 64 (s + g) + 16 j (columns past
+//      R are not stored),
+//   C:           x row i, weight rows 4 g + r for registers r.
+// Codes past the row are zeros, so a group that ends past the weights reads the last
+// super-chunk again. The sums are whole numbers: bit for bit the kernel above.
+// What bounds it is the rows: each comes from the L2 once per 64 weight rows and is quantized
+// there again. A wave keeps a whole row's loads in flight (the compiler, left to itself, waits
+// for them in small groups: 18.1 us instead of 9.2), 11 vector instructions to an element.
+// 2560 x 6912, us, here | one row a workgroup: 24 rows 9.2 | 16.3, 300 rows 44 | 159.
+// ------------------------------------------------------------------------
+typedef int rows_i4 __attribute__((ext_vector_type(4)));
+template <int R, int J>
+__global__ void __launch_bounds__(256, 2)
+tl1_rows_f32_kernel(const uint4* __restrict__ w, const float* __restrict__ x, int64_t M, int64_t N,
+                    int64_t K, int64_t KS, RowScales rs, float* __restrict__ y) {
+    extern __shared__ __align__(16) uint8_t rows_lds[];
+    const int groups = (int)((KS + 3) / 4);
+    const int stride = groups * 256 + 16;  // bytes of a row's codes: rows in different banks
+    __shared__ float inv[R];
+    __shared__ int sums[R];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int64_t b = blockIdx.x, m0 = (int64_t)blockIdx.y * R;
+    for (int r = wave; r < R && m0 + r < M; r += 4) {
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(x + (m0 + r) * K), 0, (int)(K * 4), 0x00020000);
+        float xv[J][4];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {  // groups past K read zeros (outside the resource)
+            const uint4 u = __builtin_bit_cast(
+                uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, (lane + 64 * j) * 16, 0, 0));
+            xv[j][0] = __uint_as_float(u.x);
+            xv[j][1] = __uint_as_float(u.y);
+            xv[j][2] = __uint_as_float(u.z);
+            xv[j][3] = __uint_as_float(u.w);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (all loads in flight)
+        float amax = 1e-6f;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(xv[j][e]));
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        const float scale = __fdiv_rn(31.0f, amax);
+        int csum = 0;
+        uint32_t* cs = reinterpret_cast<uint32_t*>(rows_lds + r * stride);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            int c[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[e] = act_code<31>(xv[j][e], scale);
+            if (j < groups) cs[lane + 64 * j] = pack4(c[0], c[1], c[2], c[3]);
+            csum += (c[0] + c[1]) + (c[2] + c[3]);
+        }
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) csum += __shfl_xor(csum, o, 64);
+        if (lane == 0) {
+            inv[r] = __fmul_rn(amax, 1.0f / 31.0f);
+            sums[r] = csum;
+        }
+    }
+    const int i = lane & 15, g = lane >> 4;
+    const uint4* wb = w + b * KS * 64 + i;
+    uint4 v[2][4];
+    auto load = [&](int G, uint4 (&d)[4]) {
+        const uint4* p = wb + min((int64_t)4 * G + g, KS - 1) * 64;
+#pragma unroll
+        for (int tile = 0; tile < 4; ++tile) d[tile] = p[16 * tile];
+    };
+    if (wave < groups) load(wave, v[0]);
+    __syncthreads();
+    rows_i4 acc[4] = {};
+    const uint8_t* cb = rows_lds + (i % R) * stride + 64 * g;
+    auto multiply = [&](int G, const uint4 (&d)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const rows_i4 B = *reinterpret_cast<const rows_i4*>(cb + 256 * G + 16 * j);
+#pragma unroll
+            for (int tile = 0; tile < 4; ++tile) {
+                const uint32_t wd = j == 0 ? d[tile].x : j == 1 ? d[tile].y : j == 2 ? d[tile].z : d[tile].w;
+                const rows_i4 A = {(int)(wd & 0x03030303u), (int)((wd >> 2) & 0x03030303u),
+                                   (int)((wd >> 4) & 0x03030303u), (int)((wd >> 6) & 0x03030303u)};
+                acc[tile] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, B, acc[tile], 0, 0, 0);
+            }
+        }
+    };
+    for (int G = wave; G < groups; G += 8) {
+        if (G + 4 < groups) load(G + 4, v[1]);
+        multiply(G, v[0]);
+        if (G + 8 < groups) load(G + 8, v[0]);
+        if (G + 4 < groups) multiply(G + 4, v[1]);
+    }
+    __syncthreads();  // the codes have been read
+    rows_i4* red = reinterpret_cast<rows_i4*>(rows_lds);  // [wave][x row][weight rows 4 n ..]
+    if (i < R)
+#pragma unroll
+        for (int tile = 0; tile < 4; ++tile) red[(wave * R + i) * 16 + 4 * tile + g] = acc[tile];
+    __syncthreads();
+    const int r = t >> 4, n = t & 15;
+    if (r < R && m0 + r < M) {
+        const rows_i4 tot = (red[r * 16 + n] + red[(R + r) * 16 + n]) +
+                            (red[(2 * R + r) * 16 + n] + red[(3 * R + r) * 16 + n]);
+        const int64_t row = b * 64 + 4 * n;
+        int j = 0;
+        while (j < rs.n - 1 && row >= rs.end[j]) ++j;
+        const float sc = __fmul_rn(inv[r], rs.scale[j]);
+        float* o = y + (m0 + r) * N + row;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (float)(tot[e] - sums[r]) * sc;
+    }
+}
+
+template <int R>
+static void launch_tl1_rows_f32(const uint4* w, const float* x, int64_t M, int64_t N, int64_t K,
+                                int64_t KS, const RowScales& rs, float* y, hipStream_t st) {
+    const dim3 grid((unsigned)(N / 64), (unsigned)ceil_div(M, R));
+    const size_t row = (size_t)ceil_div(KS, 4) * 256 + 16;
+    const size_t lds = R * row > 4096 * R ? R * row : 4096 * R;  // (the waves' sums: 1 KiB R)
+    if (K <= 2048)
+        hipLaunchKernelGGL((tl1_rows_f32_kernel<R, 8>), grid, dim3(256), lds, st, w, x, M, N, K, KS, rs, y);
+    else if (K <= 4096)
+        hipLaunchKernelGGL((tl1_rows_f32_kernel<R, 16>), grid, dim3(256), lds, st, w, x, M, N, K, KS, rs, y);
+    else
+        hipLaunchKernelGGL((tl1_rows_f32_kernel<R, 32>), grid, dim3(256), lds, st, w, x, M, N, K, KS, rs, y);
 }
 
 // ------------------------------------------------------------------------
@@ -916,6 +1052,20 @@ TENZO_HIP_API int tenzo_hip_bitlinear_tl1_f32(const float* x, const void* w_pack
     if (K % 4 == 0 && Kp <= 8192 && tl1_pick_splits(N / 64, KS, M) == 1) {
         const dim3 grid((unsigned)(N / 64), (unsigned)M), blk(256);
         const uint4* wp = (const uint4*)w_packed;
+        // Several rows to a workgroup once there is one for every other CU: us at 24 rows,
+        // tl1_gemv_f32_kernel | 4 rows, 2560 x 6912 16.3 | 9.2, 2560 x 2560 7.8 | 5.8; at 8 rows
+        // of 3840 x 2560 5.9 | 5.6, of 2560 x 2560 (320 one-row blocks) 5.4 | 5.6. 8 rows share
+        // the unpacked weights of many workgroups: 300 rows of 2560 x 6912 51 | 44, 48 rows of
+        // 3840 x 2560 8.7 | 9.1. Short rows quantize in no time: 2560 x 256, 24 rows 3.8 | 4.0,
+        // 48 rows 5.5 | 4.4.
+        const int64_t blocks = N / 64 * M;
+        if (M >= 4 && blocks >= (K < 1024 ? 1536 : 480)) {
+            if (blocks >= 4096)
+                launch_tl1_rows_f32<8>(wp, x, M, N, K, KS, rs, y, st);
+            else
+                launch_tl1_rows_f32<4>(wp, x, M, N, K, KS, rs, y, st);
+            return launch_status("tl1_rows_f32_kernel");
+        }
         if (Kp <= 2048)
             hipLaunchKernelGGL(tl1_gemv_f32_kernel<2>, grid, blk, 0, st, wp, x, N, K, KS, rs, y);
         else if (Kp <= 4096)

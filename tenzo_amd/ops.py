@@ -29,9 +29,9 @@ def _ptr(t: torch.Tensor | None):
     return t.data_ptr()  # (the declared argument types convert it)
 
 
-# The current stream's handle without a Stream object, views or pointer objects for nothing:
-# the small calls' kernels take 5 to 10 us, so their Python side shows. Per call, us, with
-# them | without: gemv_q4_0 10.3 | 7.3, attn_int8_decode 14.6 | 11.4, rmsnorm_quant31 + bitlinear_tl1 22.2 | 16.5.
+# The small calls' kernels take 5 to 10 us, so their Python side shows: no Stream object, pointer
+# object or view where a number or the tensor itself will do. Per call, us, with them | without:
+# gemv_q4_0 10.3 | 7.3, attn_int8_decode 14.6 | 11.4, rmsnorm_quant31 + bitlinear_tl1 22.2 | 16.5.
 def _stream() -> int:
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 

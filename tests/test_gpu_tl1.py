@@ -102,6 +102,34 @@ def test_tl1_gemv_f32_entry_bit_exact(torch_dev, N, K, M):
         np.testing.assert_array_equal(y[m], yo)
 
 
+@pytest.mark.parametrize("N,K,M", [(512, 1028, 61), (512, 2500, 64), (1024, 6912, 31),
+                                   (4096, 8192, 67), (4096, 100, 66), (64, 2052, 481)])
+def test_tl1_f32_rows_bit_exact(torch_dev, N, K, M):
+    """Rows enough for the kernel that takes 4 or 8 of them (N / 64 * M from 480 on; K < 1024 from
+    1536; 8 from 4096): row groups and groups of four super-chunks end partly filled, K is not a
+    multiple of 64. Every row equals the one-row call's bit for bit, also with an infinity or a NaN,
+    the first ones the oracle's."""
+    from tenzo_amd import ops
+    torch = torch_dev
+    rng = np.random.default_rng(N + K)
+    w = formats.tl1_random(N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[1] = 0.0
+    wp = ops.tl1_repack(to_dev(torch, w), N, K)
+    print(f"tl1_f32 rows N={N} K={K} M={M}", flush=True)
+    for m in (0, 1, M - 1):
+        yo, _, _ = oracle.tl1_gemv(x[m], w, N, 0.0159)
+        y = ops.bitlinear_tl1_f32(to_dev(torch, x), wp, 0.0159, N, K).cpu().numpy()
+        np.testing.assert_array_equal(y[m], yo)
+    x[2, K - 1] = np.inf
+    x[3, 5] = np.nan
+    xd = to_dev(torch, x)
+    y = ops.bitlinear_tl1_f32(xd, wp, 0.0159, N, K)
+    for m in range(M):
+        one = ops.bitlinear_tl1_f32(xd[m:m + 1], wp, 0.0159, N, K)
+        assert torch.equal(y[m].view(torch.int32), one[0].view(torch.int32)), m
+
+
 def test_rmsnorm_quant31_bit_exact(torch_dev):
     from tenzo_amd import ops
     torch = torch_dev
