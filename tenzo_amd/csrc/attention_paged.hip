@@ -11,12 +11,16 @@
 // one online-softmax pass:
 //   1. paged_scores_kernel  (chunk, kv head): RoPE, append, raw scores
 //      s_t = (q.k_t * s_k[t]) / sqrt(128) of the kv head's G query heads into a
-//      score buffer, and each chunk's maximum;
-//   2. paged_softmax_kernel (query head): M = max, e_t = exp(s_t - M),
-//      L = sum e_t, p_t = e_t / (L + 1e-8) in place;
-//   3. paged_values_kernel  (chunk, kv head): o_c = sum over the chunk's tokens
-//      with p_t >= 1e-7 of (p_t s_v[t]) v_t;
-//   4. paged_sum_kernel     (query head): out = sum_c o_c in chunk order.
+//      score buffer, each chunk's maximum m_c and l_c = sum of exp(s_t - m_c);
+//   2. paged_values_kernel  (chunk, kv head): M = max m_c, L = sum l_c exp(m_c - M),
+//      p_t = exp(s_t - M) / (L + 1e-8), o_c = sum over the chunk's tokens with
+//      p_t >= 1e-7 of (p_t s_v[t]) v_t;
+//   3. paged_sum_kernel     (query head): out = sum_c o_c.
+// At 8192 tokens of 20 / 5 heads the bytes (10.5 MB) take 2 us: what counts is each
+// pass's chain of memory round trips (position, block table, row; score, weight, sum).
+// So every block of 2. takes M and L from the chunks' pairs itself (a few KB, in place of
+// a pass over all scores by Hq blocks, 12.7 us) with its value rows already in flight.
+// The call: 18.1 us (four passes: 32.7), at 1000 tokens 15.7 (21.6), at 30000 34 (71).
 #include "attention.h"
 #include "common.h"
 
@@ -44,6 +48,7 @@ struct PagedArgs {
     int n_layers, layer, Hq, Hkv, T, max_chunks, score_stride;
     float* scores;  // [Hq][score_stride]
     float* cmax;    // [Hq][max_chunks]
+    float* csum;    // [Hq][max_chunks]: sums of exp(score - cmax)
     float* part;    // [Hq][max_chunks][128]
     float* out;     // [Hq][128]
 };
@@ -168,81 +173,85 @@ __global__ void __launch_bounds__(256) paged_scores_kernel(PagedArgs a) {
             m = fmaxf(m, sc[g][i]);
         }
         m = wave_max(m);
-        if (lane == 0) a.cmax[(h * G + g) * a.max_chunks + c] = m;
+        float l = 0.0f;
+        for (int i = lane; i < nt; i += 64) l += expf(sc[g][i] - m);
+        l = wave_sum_tree(l);
+        if (lane == 0) {
+            a.cmax[(h * G + g) * a.max_chunks + c] = m;
+            a.csum[(h * G + g) * a.max_chunks + c] = l;
+        }
     }
 }
 
-// Softmax of one query head over the whole context (:395-405), in place.
-__global__ void __launch_bounds__(256) paged_softmax_kernel(PagedArgs a) {
-    __shared__ float red[4];
-    __shared__ float stat;
-    const int qh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int seq_len = step_pos(a) + 1;
-    const int nchunks = (seq_len + a.T - 1) / a.T;
-    const float* cm = a.cmax + qh * a.max_chunks;
-    float M = -1e30f;
-    for (int c = 0; c < nchunks; ++c) M = fmaxf(M, cm[c]);
-    float* s = a.scores + (int64_t)qh * a.score_stride;
-    // thread tid takes t = tid, tid + 256, ... in order; a read-only pass sums
-    // the exponentials (its loads issued kU at a time), a second pass writes
-    // the normalized weights (the same expf of the same score)
-    constexpr int kU = 8;
-    float l = 0.0f;
-    for (int t0 = tid; t0 < seq_len; t0 += 256 * kU) {
-        float v[kU];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) v[u] = t0 + 256 * u < seq_len ? s[t0 + 256 * u] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < kU; ++u)
-            if (t0 + 256 * u < seq_len) l += expf(v[u] - M);
-    }
-    l = wave_sum_tree(l);
-    if (lane == 0) red[wave] = l;
-    __syncthreads();
-    if (tid == 0) stat = __fdiv_rn(1.0f, ((red[0] + red[1]) + (red[2] + red[3])) + 1e-8f);
-    __syncthreads();
-    const float inv = stat;
-    for (int t0 = tid; t0 < seq_len; t0 += 256 * kU) {
-        float v[kU];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) v[u] = t0 + 256 * u < seq_len ? s[t0 + 256 * u] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < kU; ++u)
-            if (t0 + 256 * u < seq_len) s[t0 + 256 * u] = __fmul_rn(expf(v[u] - M), inv);
-    }
-}
-
-// Weighted values of one chunk (:408-443): thread (d4, p) owns dims 4 d4 .. +3
-// of every query head and takes the chunk's tokens p, p + 8, ...
+// Softmax (:395-405) and weighted values (:408-443) of one chunk: thread (d4, p) owns dims
+// 4 d4 .. +3 of every query head and takes the chunk's tokens p, p + 8, ...
 template <int G>
 __global__ void __launch_bounds__(256) paged_values_kernel(PagedArgs a) {
+    constexpr int kU = 8;  // a thread's rows in flight
     __shared__ float ow[8][G][kD];
-    const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    __shared__ float wt[G][kMaxChunk];
+    __shared__ float stat[G][2];
+    const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int seq_len = step_pos(a) + 1;
     const int t0 = c * a.T;
     if (t0 >= seq_len) return;
     const int nt = min(a.T, seq_len - t0);
     const int nchunks = (seq_len + a.T - 1) / a.T;
     const int d4 = tid & 31, p = tid >> 5;
+    uint32_t vb[kU];
+    auto load = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            vb[u] = i0 + 8 * u < nt
+                        ? *reinterpret_cast<const uint32_t*>(
+                              a.pv + page_row(a, t0 + i0 + 8 * u, h) * kD + 4 * d4)
+                        : 0;
+    };
+    load(p);
+    for (int g = wave; g < G; g += 4) {
+        const float* cm = a.cmax + (h * G + g) * a.max_chunks;
+        const float* cl = a.csum + (h * G + g) * a.max_chunks;
+        float M = -1e30f, L = 0.0f;
+        for (int i = lane; i < nchunks; i += 64) M = fmaxf(M, cm[i]);
+        M = wave_max(M);
+        for (int i = lane; i < nchunks; i += 64) L = __builtin_fmaf(cl[i], expf(cm[i] - M), L);
+        L = wave_sum_tree(L);
+        if (lane == 0) {
+            stat[g][0] = M;
+            stat[g][1] = __fdiv_rn(1.0f, L + 1e-8f);
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < nt; i += 256) {
+        const float sv = a.pvs[page_row(a, t0 + i, h)];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float s = a.scores[(int64_t)(h * G + g) * a.score_stride + t0 + i];
+            const float alpha = __fmul_rn(expf(s - stat[g][0]), stat[g][1]);
+            wt[g][i] = alpha < 1e-7f ? 0.0f : __fmul_rn(alpha, sv);
+        }
+    }
+    __syncthreads();
     float o[G][4];
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[g][k] = 0.0f;
-    for (int i = p; i < nt; i += 8) {
-        const int t = t0 + i;
-        const int64_t r = page_row(a, t, h);
-        const uint32_t vb = *reinterpret_cast<const uint32_t*>(a.pv + r * kD + 4 * d4);
-        const float sv = a.pvs[r];
-        float vf[4];
+    for (int i0 = p; i0 < nt; i0 += 8 * kU) {
+        if (i0 != p) load(i0);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) vf[k] = (float)(int8_t)((vb >> (8 * k)) & 0xff);
+        for (int u = 0; u < kU; ++u) {
+            if (i0 + 8 * u >= nt) break;
+            float vf[4];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const float alpha = a.scores[(int64_t)(h * G + g) * a.score_stride + t];
-            const float w = alpha < 1e-7f ? 0.0f : __fmul_rn(alpha, sv);
+            for (int k = 0; k < 4; ++k) vf[k] = (float)(int8_t)((vb[u] >> (8 * k)) & 0xff);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) o[g][k] = __builtin_fmaf(w, vf[k], o[g][k]);
+            for (int g = 0; g < G; ++g) {
+                const float w = wt[g][i0 + 8 * u];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) o[g][k] = __builtin_fmaf(w, vf[k], o[g][k]);
+            }
         }
     }
 #pragma unroll
@@ -263,15 +272,17 @@ __global__ void __launch_bounds__(256) paged_values_kernel(PagedArgs a) {
     }
 }
 
-// out = sum of the chunk sums in chunk order, kSumU loads in flight.
-__global__ void __launch_bounds__(128) paged_sum_kernel(PagedArgs a) {
-    const int qh = blockIdx.x, d = threadIdx.x;
+// out = sum of the chunk sums: group q of 128 threads takes kSumU at a time, every fourth
+// run of them.
+__global__ void __launch_bounds__(512) paged_sum_kernel(PagedArgs a) {
+    __shared__ float red[4][kD];
+    const int qh = blockIdx.x, d = threadIdx.x & 127, q = threadIdx.x >> 7;
     const int seq_len = step_pos(a) + 1;
     const int nchunks = (seq_len + a.T - 1) / a.T;
     if (nchunks == 1) return;
     const float* pp = a.part + (int64_t)qh * a.max_chunks * kD + d;
     float o = 0.0f;
-    for (int c0 = 0; c0 < nchunks; c0 += kSumU) {
+    for (int c0 = q * kSumU; c0 < nchunks; c0 += 4 * kSumU) {
         float v[kSumU];
 #pragma unroll
         for (int u = 0; u < kSumU; ++u) v[u] = c0 + u < nchunks ? pp[(int64_t)(c0 + u) * kD] : 0.0f;
@@ -279,14 +290,16 @@ __global__ void __launch_bounds__(128) paged_sum_kernel(PagedArgs a) {
         for (int u = 0; u < kSumU; ++u)
             if (c0 + u < nchunks) o += v[u];
     }
-    a.out[(int64_t)qh * kD + d] = o;
+    red[q][d] = o;
+    __syncthreads();
+    if (q == 0) a.out[(int64_t)qh * kD + d] = (red[0][d] + red[1][d]) + (red[2][d] + red[3][d]);
 }
 
 }  // namespace
 
 size_t paged_ws_bytes(int Hq, int max_chunks, int T) {
     const size_t stride = (size_t)max_chunks * T;
-    return (size_t)Hq * (stride + max_chunks + (size_t)max_chunks * kD) * 4;
+    return (size_t)Hq * (stride + 2 * (size_t)max_chunks + (size_t)max_chunks * kD) * 4;
 }
 
 int launch_attn_paged(const AttnPagedLaunch& L, hipStream_t st) {
@@ -321,7 +334,8 @@ int launch_attn_paged(const AttnPagedLaunch& L, hipStream_t st) {
     if (!ws) return TENZO_ERROR_OUT_OF_MEMORY;
     a.scores = ws;
     a.cmax = ws + (size_t)L.Hq * a.score_stride;
-    a.part = a.cmax + (size_t)L.Hq * L.max_chunks;
+    a.csum = a.cmax + (size_t)L.Hq * L.max_chunks;
+    a.part = a.csum + (size_t)L.Hq * L.max_chunks;
     a.out = L.out;
     const dim3 grid(L.max_chunks, L.Hkv);
     switch (G) {
@@ -335,8 +349,6 @@ int launch_attn_paged(const AttnPagedLaunch& L, hipStream_t st) {
     }
     int rc = launch_status("paged_scores_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(paged_softmax_kernel, dim3(L.Hq), dim3(256), 0, st, a);
-    if ((rc = launch_status("paged_softmax_kernel"))) return rc;
     switch (G) {
         case 1: hipLaunchKernelGGL(paged_values_kernel<1>, grid, dim3(256), 0, st, a); break;
         case 2: hipLaunchKernelGGL(paged_values_kernel<2>, grid, dim3(256), 0, st, a); break;
@@ -345,7 +357,7 @@ int launch_attn_paged(const AttnPagedLaunch& L, hipStream_t st) {
     }
     if ((rc = launch_status("paged_values_kernel"))) return rc;
     if (L.max_chunks == 1) return TENZO_SUCCESS;
-    hipLaunchKernelGGL(paged_sum_kernel, dim3(L.Hq), dim3(128), 0, st, a);
+    hipLaunchKernelGGL(paged_sum_kernel, dim3(L.Hq), dim3(512), 0, st, a);
     return launch_status("paged_sum_kernel");
 }
 

@@ -67,6 +67,15 @@ def test_attn_paged_matches_oracle(torch_dev, Hq, Hkv, L, layer, S, pos, qs):
     assert rel(out, o_ref) < 1e-5
 
 
+@pytest.mark.parametrize("Hq,Hkv,pos,qs", [(2, 2, 63, 1.0), (4, 1, 64, 8.0), (2, 1, 4100, 1.0),
+                                           (8, 1, 9001, 30.0), (4, 2, 16500, 1.0)])
+def test_attn_paged_chunk_sums(torch_dev, Hq, Hkv, pos, qs):
+    """The softmax from the chunks' maxima and sums: one chunk, a chunk of one token, more
+    chunks than a wave has lanes and than the final sum takes at a time, scores whose
+    chunk maxima lie far apart."""
+    test_attn_paged_matches_oracle(torch_dev, Hq, Hkv, 1, 0, (pos + 16) // 16 * 16, pos, qs)
+
+
 @pytest.mark.parametrize("case", ["", "peak_"])
 def test_attn_paged_reference_fixture(torch_dev, case):
     z = np.load(os.path.join(GOLD, "attention_paged.npz"))
