@@ -97,7 +97,8 @@ TENZO_HIP_API int tenzo_hip_bitlinear_tl1_lut(const int8_t* codes, const tenzo_h
  * separate compute_from_lut calls (TenzoEngine.cpp:129-146), which
  * prefill_token (TenzoEngine.cpp:1809-1819) makes one token at a time, from
  * one pass over the packed weights: acc[m][n] and y[m][n] as in
- * tenzo_hip_bitlinear_tl1, bit for bit. tile = 0 picks the workgroup shape;
+ * tenzo_hip_bitlinear_tl1, bit for bit. tile = 0 picks the kernel and its
+ * workgroup shape for M and N;
  * 100 * KW + 10 * RW + CT forces 64*RW rows x 32*CT tokens with KW K groups
  * (142, 242, 442, 222, 422, 221, 421, 412, 411 or 811, with
  * (N/64) % RW == 0). No scratch memory is used. */
@@ -215,7 +216,8 @@ TENZO_HIP_API int tenzo_hip_gemv_q4_0_q8_0(const uint8_t* qa, const uint8_t* w, 
  * qzeros [ceil(K/g/8)][N] u32 (nibble g%8, zero = nibble + 1). B <= 8
  * rows; 9..16 with 16-byte aligned fp16 activations, K % 512 == 0,
  * g in {32, 64, 128, 256, 512} and B (K + 4) fp16 within 152 KiB (fp16 MFMA,
- * which also serves batch 4..8 of that form). */
+ * which also serves batch 4..8 of that form, in two passes or more where the
+ * rows do not fit together and K % 2048 == 0). */
 TENZO_HIP_API int tenzo_hip_gemv_gptq(const void* act, int act_dtype, const uint32_t* qweight,
                                       const void* scales, int scale_dtype,
                                       const uint32_t* qzeros, float* y, int K, int N,
@@ -310,7 +312,7 @@ struct tenzo_engine_opaque;
  * the KV cache, the hidden state and seq_len end as after n calls of
  * tenzo_prefill_token (TenzoEngine.cpp:1809-1819, C API :2187), which is how
  * the reference prefills a prompt (main_inference.cpp:470-472). Each layer
- * runs once per pass of up to 512 tokens: the TL1 projections as int8 MFMA
+ * runs once per pass of up to 2048 tokens: the TL1 projections as int8 MFMA
  * contractions (tenzo_hip_bitlinear_tl1_batch), then every token's attention
  * over its own prefix. exact != 0: the attention repeats a decode step's
  * chunking and arithmetic per token, so everything equals the per-token

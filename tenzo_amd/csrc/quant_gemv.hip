@@ -1641,19 +1641,25 @@ static int launch_gq(const TA* act, const uint32_t* qweight, const TS* scales,
                      hipStream_t st) {
     constexpr bool kF16 = std::is_same<TA, uint16_t>::value;
     // fp16 activations from batch 4 on: fp16 MFMA (K in whole 512-k chunks per part, groups of 16-k steps
-    // dividing them, the staged activations within LDS)
+    // dividing them, the staged activations within LDS). Up to 8 rows too long to be staged
+    // together go in passes over the weights where K has four parts: 8 rows of K = 14336, N = 4096,
+    // us, two passes 35.5, the packed fp16 dot below 140.5; 7 of K = 12288 33.4 and 149.6 (one part,
+    // 7 of K = 13824, N = 5120: 90.0 and 90.0, and longer sums).
+    const int fit = (int)(kGqLds / ((size_t)(K + 4) * 2));  // rows that can be staged
     if (kF16 && B >= 4 && B <= 16 && K % kGqChunk == 0 && group % 16 == 0 &&
-        kGqChunk % group == 0 && ((uintptr_t)act & 15) == 0 &&
-        (size_t)B * (K + 4) * 2 <= kGqLds) {
+        kGqChunk % group == 0 && ((uintptr_t)act & 15) == 0 && (B <= fit || (B <= 8 && fit >= 2 && K % (kGqParts * kGqChunk) == 0))) {
         int parts = kGqParts;  // K split into 4, 2 or 1 parts of whole chunks
         while (K % (parts * kGqChunk) != 0) parts /= 2;
         const dim3 grid((unsigned)ceil_div(N, 32)), block((unsigned)(128 * parts));
-        const size_t lds = (size_t)B * (K + 4) * 2;
+        const int rows = (int)ceil_div(B, ceil_div(B, fit));  // of a pass
+        const size_t lds = (size_t)rows * (K + 4) * 2;
         switch (group / 16) {
 #define GQM_CASE(NG)                                                                          \
             case NG:                                                                          \
-                hipLaunchKernelGGL((gq_mfma_kernel<AWQ, TS, NG>), grid, block, lds, st,        \
-                                   (const uint16_t*)act, qweight, scales, qzeros, y, K, N, B); \
+                for (int b = 0; b < B; b += rows)                                             \
+                    hipLaunchKernelGGL((gq_mfma_kernel<AWQ, TS, NG>), grid, block, lds, st,    \
+                                       (const uint16_t*)act + (size_t)b * K, qweight, scales,  \
+                                       qzeros, y + (size_t)b * N, K, N, B - b < rows ? B - b : rows); \
                 return launch_status(AWQ ? "awq_mfma_kernel" : "gptq_mfma_kernel");
             GQM_CASE(2) GQM_CASE(4) GQM_CASE(8) GQM_CASE(16) GQM_CASE(32)
 #undef GQM_CASE

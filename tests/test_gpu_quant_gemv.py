@@ -248,6 +248,15 @@ def test_gptq_awq_mfma_shapes(torch_dev, kind, B, K, N, G, f32s):
 
 
 @pytest.mark.parametrize("kind", ["gptq", "awq"])
+@pytest.mark.parametrize("B,K,N,G,f32s", [(6, 14336, 104, 128, False), (7, 12288, 40, 64, True),
+                                          (8, 14336, 264, 32, False), (7, 13824, 40, 128, False)])
+def test_gptq_awq_mfma_passes(torch_dev, kind, B, K, N, G, f32s):
+    """Rows too long to be staged together: passes of 3 to 4 of them over the weights, the last
+    one with fewer; K = 13824 (one K part) keeps the packed dot."""
+    test_gptq_awq_mfma_shapes(torch_dev, kind, B, K, N, G, f32s)
+
+
+@pytest.mark.parametrize("kind", ["gptq", "awq"])
 @pytest.mark.parametrize("B,K,N,G,f16a,f32s", [(1, 2048, 40, 32, True, False),
                                                (2, 6144, 1000, 64, False, True),
                                                (3, 4096, 520, 256, True, True),
