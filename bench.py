@@ -410,7 +410,7 @@ def prefill_bench(torch, e, cfg, host, args):
         "streaming_tok_s": round(n / dt, 1),
         "token_by_token_tok_s": round(seq_rate, 1),
         "speedup_vs_token_by_token": round(n / dt_exact / seq_rate, 1),
-        "roofline": {"bound": "mfma", "kernel": "tl1_mfma_kernel (gate|up projection)",
+        "roofline": {"bound": "mfma", "kernel": "tl1_mfma_wide_kernel (gate|up projection)",
                      "achieved": dom["tops"], "peak": 5000.0, "unit": "TOP/s",
                      "frac": round(dom["tops"] / 5000.0, 4), "traffic": None,
                      "rows": rows, "per_projection": roof},
