@@ -20,7 +20,7 @@
 // pass's chain of memory round trips (position, block table, row; score, weight, sum).
 // So every block of 2. takes M and L from the chunks' pairs itself (a few KB, in place of
 // a pass over all scores by Hq blocks, 12.7 us) with its value rows already in flight.
-// The call: 18.1 us (four passes: 32.7), at 1000 tokens 15.7 (21.6), at 30000 34 (71).
+// The call: 17.8 us (four passes: 32.7), at 1000 tokens 15.7 (21.6), at 30000 34 (71).
 #include "attention.h"
 #include "common.h"
 
@@ -208,14 +208,32 @@ __global__ void __launch_bounds__(256) paged_values_kernel(PagedArgs a) {
                               a.pv + page_row(a, t0 + i0 + 8 * u, h) * kD + 4 * d4)
                         : 0;
     };
+    // everything that does not wait for the softmax: the value rows, token tid's scores and
+    // value scale (a.T <= 256), the pairs of the first 128 chunks
     load(p);
+    static_assert(kMaxChunk <= 256, "one token to a thread");
+    float sv = 0.0f, sc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        sc[g] = tid < nt ? a.scores[(int64_t)(h * G + g) * a.score_stride + t0 + tid] : 0.0f;
+    if (tid < nt) sv = a.pvs[page_row(a, t0 + tid, h)];
     for (int g = wave; g < G; g += 4) {
         const float* cm = a.cmax + (h * G + g) * a.max_chunks;
         const float* cl = a.csum + (h * G + g) * a.max_chunks;
-        float M = -1e30f, L = 0.0f;
-        for (int i = lane; i < nchunks; i += 64) M = fmaxf(M, cm[i]);
+        float m[2], l[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = lane + 64 * u;
+            m[u] = i < nchunks ? cm[i] : -1e30f;
+            l[u] = i < nchunks ? cl[i] : 0.0f;
+        }
+        float M = fmaxf(fmaxf(-1e30f, m[0]), m[1]), L = 0.0f;
+        for (int i = lane + 128; i < nchunks; i += 64) M = fmaxf(M, cm[i]);
         M = wave_max(M);
-        for (int i = lane; i < nchunks; i += 64) L = __builtin_fmaf(cl[i], expf(cm[i] - M), L);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (lane + 64 * u < nchunks) L = __builtin_fmaf(l[u], expf(m[u] - M), L);
+        for (int i = lane + 128; i < nchunks; i += 64) L = __builtin_fmaf(cl[i], expf(cm[i] - M), L);
         L = wave_sum_tree(L);
         if (lane == 0) {
             stat[g][0] = M;
@@ -223,15 +241,12 @@ __global__ void __launch_bounds__(256) paged_values_kernel(PagedArgs a) {
         }
     }
     __syncthreads();
-    for (int i = tid; i < nt; i += 256) {
-        const float sv = a.pvs[page_row(a, t0 + i, h)];
+    if (tid < nt)
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const float s = a.scores[(int64_t)(h * G + g) * a.score_stride + t0 + i];
-            const float alpha = __fmul_rn(expf(s - stat[g][0]), stat[g][1]);
-            wt[g][i] = alpha < 1e-7f ? 0.0f : __fmul_rn(alpha, sv);
+            const float alpha = __fmul_rn(expf(sc[g] - stat[g][0]), stat[g][1]);
+            wt[g][tid] = alpha < 1e-7f ? 0.0f : __fmul_rn(alpha, sv);
         }
-    }
     __syncthreads();
     float o[G][4];
 #pragma unroll
