@@ -199,7 +199,10 @@ TENZO_HIP_API void tenzo_hip_rope_table(float theta, int head_dim, int pos0, int
 /* ---- Quantized GEMVs (TenzoEngine.cpp:1022-1175) ------------------------ */
 
 /* act_dtype / scale_dtype: 0 = fp32, 1 = fp16. B activation rows
- * ([B][K]), outputs [B][N] fp32. */
+ * ([B][K]), outputs [B][N] fp32. The kernel, and with it the order of a row's
+ * fp32 sums, is chosen by B, K, N and the pointers' alignment: the same row
+ * gives the same bits within one such choice, and in another batch values
+ * that differ by the rounding of those sums. */
 
 /* compute_linear_gguf_q4_0 (:1022-1075): w [N][K/32] blocks of 18 bytes. */
 TENZO_HIP_API int tenzo_hip_gemv_q4_0(const void* act, int act_dtype, const uint8_t* w,

@@ -540,31 +540,36 @@ q4_0_f16_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w,
 }
 
 // ------------------------------------------------------------------------
-// Q4_0 / Q8_0 weights times several activation rows on int8 MFMA (up to 8 rows a
+// Q4_0 / Q8_0 weights times several activation rows on bf16 MFMA (up to 8 rows a
 // workgroup; the kernels above read and unpack the weights once per row).
 //
-// y[b][n] = sum over blocks of d_n * sum_j a_bj q_nj. Per block of 32 elements the inner
-// sum is exact: a row's 32 activations become 31-bit fixed-point numbers of the block's
-// largest magnitude (a power-of-two scale s_b), in four signed byte digits, and one
-// v_mfma_i32_32x32x32_i8 multiplies them (first operand, row 8 j + b: digit j of
-// activation row b) by 32 weight rows' codes (second operand, as they are; a Q4_0 nibble
-// as 16 (q - 8)). Lane l = 32 g + n then holds weight row n's sums for activation rows
-// 4 g + e (e < 4) in registers 4 j + e, and adds d_n s_b (the digits' sums) to its fp32
-// sums: 28 vector instructions a block where products of the codes themselves take over
-// 128 for 8 rows. fp32 and fp16 activations of the same values give the same bits.
+// y[b][n] = sum over blocks of d_n * sum_j a_bj q_nj. An activation enters as the sum of
+// bf16 parts, each the truncation of what the ones before leave: three hold every bit of an
+// fp32 number, two those of an fp16 number, whatever its neighbours' magnitudes (a number
+// common to the block would take bits from small elements beside a large one). The codes are
+// exact in bf16 (a Q4_0 nibble as (q - 8) / 16), so all products are exact; two
+// v_mfma_f32_32x32x16_bf16 a block multiply the parts (first operand, row 8 j + b: part j of
+// activation row b) by 32 weight rows' codes (second operand). Lane l = 32 g + n then holds
+// weight row n's sums for activation rows 4 g + e (e < 4) in registers 4 j + e, and adds d_n
+// (the parts' sums, smallest first) to its fp32 sums. MFMA step s takes elements 16 g + 8 s ..
+// of the block from lane half g: a lane's codes are the 16 it unpacks. fp32 and fp16
+// activations of the same values give the same bits, and infinities and NaN what their
+// products give.
 //
 // A workgroup owns 32 weight rows; wave v takes blocks 8 v .. 8 v + 7 of each chunk of 8 W
-// blocks, and the waves' sums are added in LDS pairwise. Neighbouring lanes fetch
-// neighbouring 16 bytes of a row's 8 blocks (lanes that read whole blocks, or their own MFMA
-// row, cost the address unit a clock each: 1.5 and 3 times the time), one chunk ahead, and
-// leave them in the wave's LDS as they are; the chunk's digits are made once for all waves,
-// from activations that were fetched a chunk ahead too. What is left is vector work: a third
-// digits (of the same activations in every workgroup), the rest unpacking and the sums.
-// 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 19.9 | 48.1, 16 rows 36 | 113
-// (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 19.8 | 29.3.
+// blocks by itself (its activations and weights go through LDS of its own, no barriers), and
+// the waves' sums are added in LDS pairwise at the end. Neighbouring lanes fetch neighbouring
+// 16 bytes of a row's 8 blocks (lanes that read whole blocks, or their own MFMA row, cost the
+// address unit a clock each: 1.5 and 3 times the time), one chunk ahead, and leave them in
+// LDS as they are. What is left is vector work: splitting the activations (the same ones in
+// every workgroup) and converting the codes.
+// 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 17.9 | 39.2, 16 rows 27.0 | 101
+// (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 15.9 | 26.9. Error against 64 bits
+// (2-norm) of 11008 x 11008: fp32 rows 8.7e-8 | 1.3e-7, fp16 rows 8.3e-8 | 8.5e-8 (Q4_0), 8.6e-8 |
+// 8.9e-8 (Q8_0); 9.1e-8 and 9.2e-8 if a wave's chunks are one chain of sums.
 // ------------------------------------------------------------------------
-typedef int gi4 __attribute__((ext_vector_type(4)));
-typedef int gi16 __attribute__((ext_vector_type(16)));
+typedef __bf16 gb8 __attribute__((ext_vector_type(8)));
+typedef float gf16 __attribute__((ext_vector_type(16)));
 typedef uint32_t gu4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // four neighbouring activations, as loaded
@@ -573,22 +578,30 @@ struct Act4;
 template <>
 struct Act4<float> {
     typedef float4 type;
+    static constexpr int kParts = 3;
     static __device__ __forceinline__ float4 value(float4 v) { return v; }
 };
 template <>
 struct Act4<uint16_t> {
     typedef uint2 type;
+    static constexpr int kParts = 2;
     static __device__ __forceinline__ float4 value(uint2 v) {
         return make_float4(half_bits_to_float((uint16_t)v.x), half_bits_to_float((uint16_t)(v.x >> 16)),
                            half_bits_to_float((uint16_t)v.y), half_bits_to_float((uint16_t)(v.y >> 16)));
     }
 };
 
-// 16-byte unit of digit row n, half g of a block: the rows of a block (reads) and the halves
-// of a row's 8 blocks (writes) both spread over the banks, at constant distances
-constexpr int kGgBlock = 66;
-__device__ __forceinline__ int frag_unit(int blk, int g, int n) {
-    return blk * kGgBlock + g * (kGgBlock / 2) + n;
+// LDS accesses of a wave to memory of its own are performed in order; this keeps the compiler
+// from moving them across.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// two fp32 numbers' high halves (exact where the low halves are zero)
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
 template <bool Q4, typename TA, int W>  // W waves
@@ -599,10 +612,12 @@ gguf_rows_kernel(const TA* __restrict__ act, const uint8_t* __restrict__ w, floa
     constexpr int kUnits = kBytes / 2;     // 16-byte units of a row's 8 blocks
     constexpr int kLoads = (32 * kUnits + 63) / 64;
     constexpr int kChunk = 8 * W;
-    __shared__ uint4 dig[kChunk * kGgBlock];  // the chunk's digits
-    __shared__ uint4 raw[W][kLoads * 64];  // the waves' weights: [row][kUnits]
-    __shared__ __align__(16) float sa[kChunk][8];
-    __shared__ int odd_chunk;              // the last chunk with an infinity or a NaN
+    constexpr int NP = Act4<TA>::kParts;
+    // 16-byte units from one quarter of a block to the next (rows, and 2 so that the quarters
+    // and blocks that are written together lie in different banks)
+    constexpr int kQuarter = 8 * NP + 2;
+    __shared__ uint4 part[W][4 * 4 * kQuarter];  // four blocks' parts: [block][quarter][row]
+    __shared__ uint4 raw[W][kLoads * 64];        // eight blocks' weights: [row][kUnits]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, g = lane >> 5;
@@ -642,145 +657,131 @@ gguf_rows_kernel(const TA* __restrict__ act, const uint8_t* __restrict__ w, floa
         }
     };
 
-    // activations: thread tid takes elements 4 (tid % 8) .. + 3 of the chunk's block tid / 8
-    const int ablk = tid >> 3, l8 = tid & 7;
+    // activations: of four blocks, this lane takes elements 4 (lane % 8) .. + 3 of block
+    // lane / 16, rows 2 q + lane / 8 % 2
+    const int ablk = lane >> 4, rb = lane >> 3 & 1, l8 = lane & 7;
     typedef typename Act4<TA>::type Act;
-    Act x[8];
-    auto load_acts = [&](int bk0) {
-        const bool in = bk0 + ablk < nbk;
+    Act x[2][4];
+    auto load_acts = [&](int bk, Act (&v)[4]) {  // blocks bk .. bk + 3
+        const bool in = bk + ablk < nbk;
 #pragma unroll
-        for (int b = 0; b < 8; ++b)
-            x[b] = in && b < nb ? *reinterpret_cast<const Act*>(act + (int64_t)b * K +
-                                                                (bk0 + ablk) * 32 + 4 * l8)
+        for (int q = 0; q < 4; ++q) {
+            const int b = 2 * q + rb;
+            v[q] = in && b < nb ? *reinterpret_cast<const Act*>(act + (int64_t)b * K +
+                                                                (bk + ablk) * 32 + 4 * l8)
                                 : Act{};
+        }
     };
-    auto store_digits = [&](int bk0) {
-        uint32_t* o = reinterpret_cast<uint32_t*>(dig);
+    char* const pw = reinterpret_cast<char*>(part[wave]) +
+                     ((ablk * 4 + (l8 >> 1)) * kQuarter + rb) * 16 + 8 * (l8 & 1);
+    auto store_parts = [&](const Act (&v)[4]) {
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            if (b >= nb) break;  // (uniform; idle rows' sums are not stored)
-            const float4 xb = Act4<TA>::value(x[b]);
-            const float v[4] = {xb.x, xb.y, xb.z, xb.w};
-            uint32_t mb = 0;  // the largest |x|, as bits (infinities and NaN on top)
+        for (int q = 0; q < 4; ++q) {
+            if (2 * q >= nb) break;  // (uniform; idle rows' sums are not stored)
+            const float4 xq = Act4<TA>::value(v[q]);
+            float r[4] = {xq.x, xq.y, xq.z, xq.w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) mb = max(mb, __float_as_uint(v[e]) & 0x7fffffffu);
-            mb = max(mb, (uint32_t)dpp_i<kDppXor1>((int)mb));
-            mb = max(mb, (uint32_t)dpp_i<kDppXor2>((int)mb));
-            mb = max(mb, (uint32_t)dpp_i<kDppHalfMirror>((int)mb));
-            // the largest |x| 2^sh in [2^29, 2^30): within the four digits' range
-            const bool fin = mb < 0x7f800000u;
-            const int sh = min(30 - __builtin_amdgcn_frexp_expf(__uint_as_float(mb)), 145);
-            uint32_t t[4];
+            for (int j = 0; j < NP; ++j) {
+                *reinterpret_cast<uint2*>(pw + (8 * j + 2 * q) * 16) =
+                    make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3]));
+                if (j + 1 < NP) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                t[e] = (uint32_t)(int)__builtin_amdgcn_ldexpf(v[e], sh) + 0x80808080u;
-            const uint32_t a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);
-            const uint32_t a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
-            const uint32_t c01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);
-            const uint32_t c23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
-            const uint32_t dg[4] = {__builtin_amdgcn_perm(c23, c01, 0x07060302u),
-                                    __builtin_amdgcn_perm(c23, c01, 0x05040100u),
-                                    __builtin_amdgcn_perm(a23, a01, 0x07060302u),
-                                    __builtin_amdgcn_perm(a23, a01, 0x05040100u)};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o[4 * frag_unit(ablk, l8 >> 2, 8 * j + b) + (l8 & 3)] = dg[j] ^ 0x80808080u;
-            if (l8 == 0) {
-                sa[ablk][b] = fin ? __builtin_amdgcn_ldexpf(1.0f, -sh - (Q4 ? 4 : 0))
-                                  : __uint_as_float(0x7fc00000u);
-                if (!fin) odd_chunk = bk0;
+                    for (int e = 0; e < 4; ++e) {
+                        const float h = __uint_as_float(__float_as_uint(r[e]) & 0xffff0000u);
+                        r[e] = j == 0 && r[e] == h ? 0.0f : r[e] - h;  // (an infinity leaves nothing)
+                    }
+                }
             }
         }
     };
 
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // activation rows 4 g + e
-    if (tid == 0) odd_chunk = -1;
-    for (int i = tid; i < kChunk * 8; i += 64 * W) sa[i >> 3][i & 7] = 0.0f;
-    load_acts(0);
-    load_codes(8 * wave);
-    __syncthreads();
-    for (int bk0 = 0; bk0 < nbk; bk0 += kChunk) {
-        const int bk = bk0 + 8 * wave;
-        store_digits(bk0);
+    const uint4* const pr = part[wave] + 2 * g * kQuarter + (n < 8 * NP ? n : n - 8);
+    const uint32_t* const wr = reinterpret_cast<const uint32_t*>(&raw[wave][n * kUnits]);
+    gf16 zero{};  // (kept in registers: a constant is moved into them for every block)
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) raw[wave][lane + 64 * i] = wq[i];
-        if (bk0 + kChunk < nbk) {
-            load_acts(bk0 + kChunk);
-            load_codes(bk + kChunk);
+    for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(zero[e]));
+    // The sums and the weight scale of block 4 h + i, its parts at pr. Even blocks start on a
+    // word with their scale; odd ones have their codes on words, and the scale before them
+    auto product = [&](int h, int i, float (&f)[4]) {
+        const int at = kBytes * h + ((kBytes * i) >> 2), c = at + (i & 1) + (Q4 ? 0 : 4 * g);
+        uint32_t q[4] = {wr[c], wr[c + 1], wr[c + 2], wr[c + 3]};
+        if (!(i & 1)) {
+            const uint32_t v = wr[c + 4];
+            q[0] = __builtin_amdgcn_alignbyte(q[1], q[0], 2);
+            q[1] = __builtin_amdgcn_alignbyte(q[2], q[1], 2);
+            q[2] = __builtin_amdgcn_alignbyte(q[3], q[2], 2);
+            q[3] = __builtin_amdgcn_alignbyte(v, q[3], 2);
         }
-        __syncthreads();
-        const bool slow = odd_chunk == bk0;
-        const int m = min(8, nbk - bk);
-        const uint32_t* wr = reinterpret_cast<const uint32_t*>(&raw[wave][n * kUnits]);
-        // block j's sums and weight scale. Even blocks start on a word with their scale; odd
-        // ones have their codes on words, and the scale before them
-        auto product = [&](int j4, int i, float (&f)[4]) {  // block j4 + i, j4 % 4 == 0
-            const int blk = 8 * wave + j4 + i;
-            const uint4 au = dig[frag_unit(blk, g, n)];
-            const float4 s4 = *reinterpret_cast<const float4*>(&sa[blk][4 * g]);
-            const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
-            const int at = kBytes * j4 / 4 + ((kBytes * i) >> 2), c = at + (i & 1) + (Q4 ? 0 : 4 * g);
-            uint32_t q[4] = {wr[c], wr[c + 1], wr[c + 2], wr[c + 3]};
-            if (!(i & 1)) {
-                const uint32_t x = wr[c + 4];
-                q[0] = __builtin_amdgcn_alignbyte(q[1], q[0], 2);
-                q[1] = __builtin_amdgcn_alignbyte(q[2], q[1], 2);
-                q[2] = __builtin_amdgcn_alignbyte(q[3], q[2], 2);
-                q[3] = __builtin_amdgcn_alignbyte(x, q[3], 2);
-            }
-            if (Q4) {  // elements 0..15 in the low nibbles (g = 0), 16..31 in the high
+        if (Q4) {  // elements 0..15 in the low nibbles (g = 0), 16..31 in the high
 #pragma unroll
-                for (int k = 0; k < 4; ++k) q[k] = ((q[k] << (g ? 0 : 4)) & 0xf0f0f0f0u) ^ 0x80808080u;
-            }
-            const gi16 r = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                gi4{(int)au.x, (int)au.y, (int)au.z, (int)au.w},
-                gi4{(int)q[0], (int)q[1], (int)q[2], (int)q[3]}, gi16{}, 0, 0, 0);
+            for (int k = 0; k < 4; ++k) q[k] = (q[k] >> (4 * g)) ^ 0x08080808u;
+        }
+        uint32_t cv[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float v[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                f[e] = sc[e] * __builtin_fmaf((float)((r[e] << 8) + r[4 + e]), 65536.0f,
-                                              (float)((r[8 + e] << 8) + r[12 + e]));
-            return half_bits_to_float((uint16_t)(i & 1 ? wr[at] >> 16 : wr[at] & 0xffffu));
-        };
-        // a chunk's blocks are added pairwise: short chains of fp32 sums (m is even)
+                v[e] = Q4 ? __builtin_amdgcn_cvt_off_f32_i4((int)(q[k] >> (8 * e)))
+                          : (float)(int8_t)(q[k] >> (8 * e));
+            cv[2 * k] = bf16_pair(v[0], v[1]);
+            cv[2 * k + 1] = bf16_pair(v[2], v[3]);
+        }
+        gf16 r = zero;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            r = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(gb8, pr[(4 * i + s) * kQuarter]),
+                __builtin_bit_cast(gb8, uint4{cv[4 * s], cv[4 * s + 1], cv[4 * s + 2], cv[4 * s + 3]}),
+                r, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = NP == 3 ? (r[8 + e] + r[4 + e]) + r[e] : r[4 + e] + r[e];
+        const float d = half_bits_to_float((uint16_t)(i & 1 ? wr[at] >> 16 : wr[at] & 0xffffu));
+        return Q4 ? 16.0f * d : d;
+    };
+
+    float acc[4] = {}, run[4] = {};  // activation rows 4 g + e; the last 1 to 4 chunks apart
+    int nrun = 0;
+    load_acts(8 * wave, x[0]);
+    load_acts(8 * wave + 4, x[1]);
+    load_codes(8 * wave);
+    for (int bk = 8 * wave; bk < nbk; bk += kChunk) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) raw[wave][lane + 64 * i] = wq[i];
+        load_codes(bk + kChunk);
+        const int m = min(8, nbk - bk);
         float sum[4] = {};
-#pragma unroll 1
-        for (int j = 0; j < m; j += 4) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (4 * h >= m) break;
+            store_parts(x[h]);
+            load_acts(bk + kChunk + 4 * h, x[h]);
+            wave_lds_order();
+            // the blocks are added pairwise: short chains of fp32 sums (m is even)
             float f[4][4], d[4];
-            d[0] = product(j, 0, f[0]), d[1] = product(j, 1, f[1]);
-            if (j + 4 <= m)
-                d[2] = product(j, 2, f[2]), d[3] = product(j, 3, f[3]);
+            d[0] = product(h, 0, f[0]), d[1] = product(h, 1, f[1]);
+            if (4 * h + 4 <= m)
+                d[2] = product(h, 2, f[2]), d[3] = product(h, 3, f[3]);
             else
                 for (int e = 0; e < 4; ++e) f[2][e] = f[3][e] = d[2] = d[3] = 0.0f;
-            if (slow) {  // (uniform) blocks with an infinity or a NaN: their products one by one
-                const int8_t* wb = reinterpret_cast<const int8_t*>(wr);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int blk = j + (i >> 2), b = 4 * g + (i & 3);
-                    const float sc = sa[8 * wave + blk][b];
-                    if (blk >= m || sc == sc) continue;
-                    float p = 0.0f;
-#pragma unroll 1
-                    for (int k = 0; k < 32; ++k) {
-                        const int8_t* c = wb + kBytes * blk + 2;
-                        const float q = Q4 ? (float)((c[k & 15] >> (k & 16 ? 4 : 0)) & 15) - 8.0f
-                                           : (float)c[k];
-                        p = __builtin_fmaf(to_f32<TA>(act[(int64_t)b * K + (bk + blk) * 32 + k]), q, p);
-                    }
-                    f[i >> 2][i & 3] = p;
-                }
-            }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 sum[e] += __builtin_fmaf(f[1][e], d[1], f[0][e] * d[0]) +
                           __builtin_fmaf(f[3][e], d[3], f[2][e] * d[2]);
+            wave_lds_order();
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += sum[e];
-        __syncthreads();  // the chunk has been read
-    }
-    float* red = reinterpret_cast<float*>(dig);  // [wave][activation row][weight row]
+        for (int e = 0; e < 4; ++e) run[e] += sum[e];
+        if (++nrun == 4) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[(wave * 8 + 4 * g + e) * 32 + n] = acc[e];
+            for (int e = 0; e < 4; ++e) acc[e] += run[e], run[e] = 0.0f;
+            nrun = 0;
+        }
+    }
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(part);  // [wave][activation row][weight row]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[(wave * 8 + 4 * g + e) * 32 + n] = acc[e] + run[e];
     __syncthreads();
     if (tid < 256) {
         const int b = tid >> 5;

@@ -116,14 +116,14 @@ def test_q8_0_weights(torch_dev, N, K, B):
     np.testing.assert_array_equal(y32, y)  # the same fp32 activations either way
 
 
-@pytest.mark.parametrize("N,K,B", [(8191, 64, 2), (5504, 3200, 9), (4097, 2304, 8),
+@pytest.mark.parametrize("N,K,B", [(8191, 320, 2), (5504, 3200, 9), (4097, 2304, 8),
                                    (8225, 4096, 17), (16400, 448, 4), (2049, 576, 4)])
 @pytest.mark.parametrize("kind", ["q4_0", "q8_0"])
 def test_gguf_several_rows(torch_dev, kind, N, K, B):
     """Rows enough for the matrix-core kernel: row tiles, chunks and the segments of 8 blocks
     end partly filled (N % 32, K % 256 and K % 2048 != 0), groups of 8 activation rows too, with
-    four and eight waves. The sums are exact but for their fp32 additions, at most
-    K / 32 + 16 roundings of partial sums of at most sum |a w|. A row whose blocks hold an
+    four and eight waves. The products are exact and their sums are at most K / 32 + 16 fp32
+    roundings of partial sums of at most sum |a w| (wide fp32 blocks: the next test). A row whose blocks hold an
     infinity or a NaN gives what its products give, and leaves the others alone."""
     from tenzo_amd import ops
     torch = torch_dev
@@ -156,6 +156,41 @@ def test_gguf_several_rows(torch_dev, kind, N, K, B):
         last = np.float64(np.inf) * W[:, K - 1]  # (NaN where the code is 0)
     np.testing.assert_array_equal(z[0], last)
     np.testing.assert_array_equal(z[2:], y16[2:])
+
+
+@pytest.mark.parametrize("N,K,B", [(8192, 3200, 1), (16390, 320, 1), (4097, 576, 3), (8200, 4096, 8),
+                                   (2048, 14336, 16)])
+@pytest.mark.parametrize("kind", ["q4_0", "q8_0"])
+def test_gguf_rows_wide_blocks(torch_dev, kind, N, K, B):
+    """One large activation in every block, under weights whose code there is 0: the others
+    count with all their bits. fp32 rows with full mantissas, factors up to 2^66, and fp16 rows.
+    Products are exact; about 20 roundings of 2^-24 lie on a term's way through the sums, and as
+    their signs are independent the 2-norm of the error is below sqrt(20) 2^-24 < 2.7e-7 of
+    that of the result (12288 sums at least: the share hardly varies)."""
+    from tenzo_amd import ops
+    torch = torch_dev
+    rng = np.random.default_rng(N + K + B)
+    d = (0.002 + 0.004 * rng.random((N, K // 32))).astype(np.float16)
+    spot = 32 * np.arange(K // 32) + rng.integers(0, 32, K // 32)
+    if kind == "q4_0":
+        q = rng.integers(0, 16, size=(N, K), dtype=np.uint8)
+        q[:, spot] = 8
+        w, W = formats.q4_0_pack(q, d), q4_dense(q, d)
+    else:
+        q = rng.integers(-128, 128, size=(N, K)).astype(np.int8)
+        q[:, spot] = 0
+        w, W = formats.q8_0_pack(q, d), q.astype(np.float64) * np.repeat(d.astype(np.float64), 32, axis=1)
+    w, W = dev(torch, w), torch.from_numpy(W).cuda()
+    run = getattr(ops, "gemv_" + kind)
+    for factor, dtype in ((1.0, torch.float32), (1e3, torch.float32), (1e6, torch.float32),
+                          (2.0 ** 66, torch.float32), (1e3, torch.float16), (3e4, torch.float16)):
+        print(f"{kind} N={N} K={K} B={B} factor={factor} {dtype}", flush=True)
+        a = rng.standard_normal((B, K)).astype(np.float32)
+        a[:, spot] = factor
+        a = dev(torch, a).to(dtype)
+        y = run(a, w, K, N).double()
+        ref = a.double() @ W.T
+        assert ((y - ref).norm() / ref.norm()).item() < 2.7e-7, factor
 
 
 @pytest.mark.parametrize("N,K", [(64, 32), (11008, 4096), (100, 2304), (257, 8192), (33, 288)])
