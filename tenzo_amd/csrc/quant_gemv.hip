@@ -1552,23 +1552,42 @@ static int pick_lpr(int ngroups) {
 }
 
 // gguf_rows_kernel where it is the faster one. It needs words at every second block
-// (K % 64 == 0) and aligned activations. Its time hardly depends on B, that of the kernels
-// above is B rows' unpacking: us at N x K = 4096 x 4096, here | above, 4 rows 10.8 | 12.4 (Q8_0)
-// and 8.8 | 11.3 (Q4_0, fp32), 2 rows 9.7 | 8.0 and 8.1 | 7.4; fp16 rows times Q4_0 are products
-// of half pairs there: 8 rows 11.0 | 12.3, 4 rows 9.0 | 7.2, and over 8192 weight rows 3 rows
-// 26.1 | 24.9, 4 rows 26.8 | 32.6 (22016 x 4096). Without whole groups of 8 blocks the kernels
-// above take two bytes at a time: 2 rows, 5504 x 3200, 9.4 | 22.7 (Q8_0), 7.8 | 66.8 (Q4_0,
-// fp32), 7.9 | 11.9 (Q4_0, fp16). Eight waves a workgroup while each has a CU to itself
-// (8192 x 4096, 8 rows: 15.1, four waves 19.7), else four, two to a CU (14336: 22.6, eight 27.1).
+// (K % 64 == 0) and aligned activations. Its time grows by the weights, that of the kernels
+// above by B rows' unpacking; us, here | above:
+//  * whole groups of 8 blocks: from 16384 sums of two rows on (4096 x 4096, Q8_0 fp16: 4 rows
+//    8.8 | 10.2, 2 rows 8.5 | 6.5; 11008 x 2560 2 rows 11.5 | 13.3, Q4_0 fp32 11.2 | 14.5), for
+//    Q4_0 fp32 not over short rows (20000 x 512: 2 rows 7.7 | 6.6). Two rows of K = 4096 stay
+//    above where a second workgroup falls to some of the CUs only (9216 x 4096: Q8_0 15.4 |
+//    13.3, Q4_0 14.0 | 13.3; 12288: Q8_0 16.6 | 17.5).
+//  * fp16 rows times Q4_0 are products of half pairs there: from 32768 sums of four rows on
+//    (4096 x 4096: 8 rows 9.5 | 11.8, 4 rows 8.5 | 7.3; 4096 x 1024: 8 rows 5.7 | 5.1, 9 rows
+//    5.8 | 6.2; 4096 x 512: 8 rows 5.7 | 4.0).
+//  * else the kernels above take two bytes at a time: 2 rows of 11008 x 3200 14.2 | 39.7 (Q8_0),
+//    12.6 | 130 (Q4_0, fp32), 12.2 | 21.6 (Q4_0, fp16). Short rows of a tall matrix are
+//    cheap there, as a workgroup here costs 1.5 us whatever K is: one row of 32000 x 576 9.6 |
+//    9.0 (Q8_0), of 50000 x 192 13.8 | 5.0, 12.8 | 5.9 (Q4_0, fp32) and 10.0 | 3.9 (Q4_0, fp16),
+//    two of 8192 x 192 4.9 | 5.0, 4.6 | 5.9 and 4.6 | 3.9.
+// Eight waves a workgroup while each has a CU to itself (Q8_0 fp16, 8 rows of 8192 x 4096: 12.0,
+// four waves 13.8), else four, two to a CU (14336 x 4096: 19.9, eight 23.3).
+template <bool Q4, typename TA>
+static bool gguf_rows_faster(int K, int N, int B, bool full) {
+    constexpr bool kPairs = Q4 && sizeof(TA) == 2, kQ4F32 = Q4 && !kPairs;
+    const int64_t sums = (int64_t)B * N, groups = ceil_div(N, 32) * ceil_div(B, 8);
+    if (!full) {
+        if (sums < (kPairs ? 8192 : 4096)) return false;
+        if (K < 320) return kQ4F32 && K >= 128 && groups <= 512;
+        return N <= (kQ4F32 ? 104 : 55) * (int64_t)B * K;
+    }
+    if (kPairs) return B >= 4 && K >= 768 && sums >= (K < 1280 ? 36864 : 32768);
+    if (B < 2 || sums < 16384 || (Q4 && K < (B < 4 ? 768 : 512))) return false;
+    return !(B == 2 && K >= 4096 && K < 5120 && groups > 256 && groups <= (Q4 ? 320 : 352));
+}
+
 template <bool Q4, typename TA>
 static bool launch_gguf_rows(const TA* act, const uint8_t* w, float* y, int K, int N, int B,
                              hipStream_t st) {
     if (K % 64 != 0 || ((uintptr_t)w & 3) != 0 || ((uintptr_t)act & 15) != 0) return false;
-    constexpr bool kPairs = Q4 && sizeof(TA) == 2;
-    const bool full = K % 256 == 0 && ((uintptr_t)w & 15) == 0;
-    const int64_t sums = (int64_t)B * N;
-    if (full ? sums < (kPairs ? 32768 : 16384) || B < (kPairs ? 4 : 2) : sums < (kPairs ? 8192 : 4096))
-        return false;
+    if (!gguf_rows_faster<Q4, TA>(K, N, B, K % 256 == 0 && ((uintptr_t)w & 15) == 0)) return false;
     const dim3 grid((unsigned)ceil_div(N, 32), (unsigned)ceil_div(B, 8));
     if ((int64_t)grid.x * grid.y <= 256)
         hipLaunchKernelGGL((gguf_rows_kernel<Q4, TA, 8>), grid, dim3(512), 0, st, act, w, y, K, N, B);
