@@ -353,8 +353,10 @@ TENZO_HIP_API int tenzo_hip_engine_set_rope_theta(struct tenzo_engine_opaque* e,
 TENZO_HIP_API int tenzo_hip_engine_get_logits(struct tenzo_engine_opaque* e, float* logits);
 /* Copies an engine buffer to host memory, by name: "x" (hidden state),
  * "qkv" (pre-RoPE q | k | v), "attn_out", "h1", "gate_up" (gate | up),
- * "logits" - the last layer's values of the last step. n is the capacity of
- * out in floats. */
+ * "logits" - the last layer's values of the last step; "prefill_qkv" and
+ * "prefill_attn" - the last layer's q | k | v and attention output, a row per
+ * token, of the last batched-prefill pass (none before the first). n is the
+ * capacity of out in floats. */
 TENZO_HIP_API int tenzo_hip_engine_get_buffer(struct tenzo_engine_opaque* e, const char* name,
                                               float* out, int64_t n);
 /* Per-layer state of the last step when it ran the persistent kernel (mode 2),

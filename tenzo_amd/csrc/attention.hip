@@ -1272,13 +1272,13 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(AttnArgs a) {
 // waves share a row half's key tiles of 32 tokens (group k: tiles k, k + KG, ...). Each
 // round of KG tiles is laid out in LDS once for the waves of both halves (the 16-row kernel
 // above loads and converts every code once per 16 rows, and keeps the row statistics in
-// 16-lane butterflies). A round is bound by the vector unit: ~380 instructions a wave
-// beside 28 MFMAs.
+// 16-lane butterflies). A round is bound by the vector unit: ~400 instructions a wave
+// beside 32 MFMAs.
 //
-// Scores, S^T = K Q^T on v_mfma_i32_32x32x32_i8: the cache codes are the operand as they
-// are, and a query row enters as a 24-bit fixed-point number of its largest |q| in three
-// signed byte digits, so the sums are whole numbers and exact (fp16 hi + lo parts carry 22
-// bits and need the codes converted). Lane l = 32g + n holds row n's scores of tokens
+// Scores, S^T = K Q^T on v_mfma_f32_32x32x16_f16 of exact products: the codes in fp16 and
+// a query row as the 16-row kernel has it, fp16 hi + lo parts of its power-of-two multiple,
+// the lo parts' products first (a row's elements as whole numbers of its largest |q| hold small
+// ones in fewer bits, and lose NaN). Lane l = 32g + n holds row n's scores of tokens
 // 8a + 4g + b in register 4a + b: a row's maximum and sum are one lane's registers and one
 // exchange with lane l ^ 32, and its weights are already the second operand of
 // O^T = V^T W^T if k slot (g, 4a' + b) of step s means token 16s + 8a' + 4g + b.
@@ -1287,32 +1287,15 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(AttnArgs a) {
 // fp32 (left in the MFMA's accumulator over a prefix, the sums drift: it does not round to
 // nearest).
 //
-// LDS, a tile: K token t's 16-byte piece p at place p ^ (t / 2 % 8) of its 128 bytes; V^T
+// LDS, a tile: K token t's 16-byte piece p at place p ^ (t % 16) of its 256 bytes; V^T
 // dim d at row d ^ (d / 16 % 4) (the low two bits), its piece (s, g) at place
 // (2s + g) ^ (d / 4 % 4) of 64 bytes. The 16 lanes that a read serves together touch the
 // 64 banks once each, and a write's 32 lanes twice.
 constexpr int kFlashRows = 64;
-constexpr int kFlashTile = 4096 + 8192;  // K codes, V^T in fp16
+constexpr int kFlashTile = 8192 + 8192;  // K and V^T in fp16
 
 typedef _Float16 h8a __attribute__((ext_vector_type(8)));
 typedef float f16a __attribute__((ext_vector_type(16)));
-typedef int i16a __attribute__((ext_vector_type(16)));
-typedef int i4a __attribute__((ext_vector_type(4)));
-
-// The three signed byte digits of four fixed-point numbers |w| <= 0x7f7f7f, most significant
-// first: byte i of digit j is number i's.
-__device__ __forceinline__ void digits4(const int (&w)[4], int (&dig)[3]) {
-    uint32_t t[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t[i] = (uint32_t)w[i] + 0x808080u;  // bytes: digit + 128
-    const uint32_t a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);  // bytes 0, 0, 1, 1
-    const uint32_t a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
-    const uint32_t c01 = __builtin_amdgcn_perm(t[1], t[0], 0x06020602u);  // byte 2 of both
-    const uint32_t c23 = __builtin_amdgcn_perm(t[3], t[2], 0x06020602u);
-    dig[2] = (int)(__builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u);
-    dig[1] = (int)(__builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x80808080u);
-    dig[0] = (int)(__builtin_amdgcn_perm(c23, c01, 0x05040100u) ^ 0x80808080u);
-}
 
 template <int G, int KG>
 __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArgs a) {
@@ -1401,33 +1384,29 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
     }
     __syncthreads();
 
-    // the rows' digits: step s, dims 32 s + 16 g ..; the largest |q| scaled to [2^22, 2^23),
-    // or half of that where it would pass the digits' range
-    i4a qd[4][3];
+    // the rows' parts: step s, dims 16 s + 8 g ..
+    h8a qh[8], ql[8];
     float c2, qin;  // (qin: a score's unit; c2: the same times log2(e))
     {
-        const float* qrow = qs + (rg * 32 + n) * kQS + 16 * g;
+        const float* qrow = qs + (rg * 32 + n) * kQS + 8 * g;
         float mx = 0.0f;
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 8; ++s)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) mx = fmaxf(mx, fabsf(qrow[32 * s + e]));
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(qrow[16 * s + e]));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        int sh = fp16_span_exp(mx) + 9;
-        if (ldexpf(mx, sh) > 8355711.0f) --sh;
+        const int sh = fp16_span_exp(mx);
         const float up = ldexpf(1.0f, sh);
         qin = ldexpf(1.0f, -sh);
         c2 = 1.44269502f * qin;
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 8; ++s)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                int w[4], dig[3];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) w[i] = (int)rintf(qrow[32 * s + 4 * e + i] * up);
-                digits4(w, dig);
-#pragma unroll
-                for (int j = 0; j < 3; ++j) qd[s][j][e] = dig[j];
+            for (int e = 0; e < 8; ++e) {
+                const float xs = qrow[16 * s + e] * up;  // (exact: a power of two)
+                const _Float16 hi = (_Float16)xs;
+                qh[s][e] = hi;
+                ql[s][e] = (_Float16)(xs - (float)hi);
             }
     }
     const int qi = (rg * 32 + n) / G;
@@ -1439,33 +1418,28 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) o[dt] = f16a{};
     const char* kt = buf + kg * kFlashTile;
-    const char* vt = kt + 4096;
-    const uint32_t koff = (uint32_t)n * 128u, kswz = (uint32_t)((g ^ (n >> 1 & 7)) * 16);
+    const char* vt = kt + 8192;
+    const uint32_t koff = (uint32_t)n * 256u, kswz = (uint32_t)((g ^ (n & 15)) * 16);
     const uint32_t voff = (uint32_t)((n & 28) | ((n ^ (n >> 4)) & 3)) * 64u;
     const uint32_t vswz = (uint32_t)((g ^ (n >> 2 & 3)) * 16);
 
     auto step = [&](int t0, bool masked) {
-        i16a d0{}, d1{}, d2{};
+        f16a d{};
+        h8a k[8];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const i4a k = *reinterpret_cast<const i4a*>(kt + koff + (kswz ^ (uint32_t)(2 * s * 16)));
-            d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][0], d0, 0, 0, 0);
-            d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][1], d1, 0, 0, 0);
-            d2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, qd[s][2], d2, 0, 0, 0);
+        for (int s = 0; s < 8; ++s) {
+            k[s] = *reinterpret_cast<const h8a*>(kt + koff + (kswz ^ (uint32_t)(2 * s * 16)));
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[s], ql[s], d, 0, 0, 0);
         }
-        f16a d;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) d = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[s], qh[s], d, 0, 0, 0);
         float mx = -1e30f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const float4 f = *reinterpret_cast<const float4*>(&ksl[kg][8 * q + 4 * g]);
             const float fs[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = 4 * q + e;
-                const float dot = __builtin_fmaf((float)d0[j], 65536.0f,
-                                                 (float)((d1[j] << 8) + d2[j]));
-                d[j] = __fmul_rn(dot, fs[e]);
-            }
+            for (int e = 0; e < 4; ++e) d[4 * q + e] = __fmul_rn(d[4 * q + e], fs[e]);
         }
         if (masked) {  // (uniform: the tiles on the diagonal and past it)
 #pragma unroll
@@ -1496,14 +1470,18 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 ls += d[4 * q + e];
-                float w = __fmul_rn(d[4 * q + e], fs[e]);  // (fs: s_v 2^e)
-                // (opaque: fused with the product, one of hi's two uses would round once
-                // instead of twice, and lo would not be its remainder on a tie)
-                asm("" : "+v"(w));
-                const _Float16 hi = (_Float16)w;
-                wh[q >> 1][4 * (q & 1) + e] = hi;
-                wl[q >> 1][4 * (q & 1) + e] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, w);
+                d[4 * q + e] = __fmul_rn(d[4 * q + e], fs[e]);  // (fs: s_v 2^e)
             }
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            // (opaque: fused with the product, one of hi's two uses would round once
+            // instead of twice, and lo would not be its remainder on a tie)
+            float w = d[j];
+            asm("" : "+v"(w));
+            const _Float16 hi = (_Float16)w;
+            wh[j >> 3][j & 7] = hi;
+            wl[j >> 3][j & 7] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, w);
         }
         lr = __builtin_fmaf(lr, rs, ls);
         const float dn = vdn[kg];
@@ -1542,7 +1520,7 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
     uint32_t e64 = 0x64006400u;  // (a VGPR operand of v_perm_b32)
     asm volatile("" : "+v"(e64));
     const h2a bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const uint32_t kw = (uint32_t)((ti >> 3) * 128 + ((ti & 7) ^ (ti >> 4 & 7)) * 16);
+    const uint32_t kw = (uint32_t)((ti >> 3) * 256 + ((2 * (ti & 7)) ^ (ti >> 3 & 15)) * 16);
     // V: dims 4 c + f (c = ti % 32) of tokens 4 Q .. (Q = ti / 32): 8 bytes of piece (s, g)
     const int vQ = ti >> 5, vc = ti & 31;
     const uint32_t vw = (uint32_t)(vc * 256 + ((2 * (vQ >> 2) + (vQ & 1)) ^ (vc & 3)) * 16 +
@@ -1553,7 +1531,10 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
             char* tk = buf + (2 * tx + x) * kFlashTile;
-            *reinterpret_cast<uint4*>(tk + kw) = kr[x];
+            const h4a k0 = i8x4_h4(kr[x].x, e64), k1 = i8x4_h4(kr[x].y, e64);
+            const h4a k2 = i8x4_h4(kr[x].z, e64), k3 = i8x4_h4(kr[x].w, e64);
+            *reinterpret_cast<h8a*>(tk + kw) = __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
+            *reinterpret_cast<h8a*>(tk + (kw ^ 16u)) = __builtin_shufflevector(k2, k3, 0, 1, 2, 3, 4, 5, 6, 7);
             uint32_t v[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = vr[x][e] ^ 0x80808080u;
@@ -1568,7 +1549,7 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
                     __builtin_bit_cast(h2a, __builtin_amdgcn_perm(e64, f < 2 ? t01a : t01b, sel)) + bias;
                 const h2a p23 =
                     __builtin_bit_cast(h2a, __builtin_amdgcn_perm(e64, f < 2 ? t23a : t23b, sel)) + bias;
-                *reinterpret_cast<h4a*>(tk + 4096 + vw + ((f ^ (vc >> 2)) & 3) * 64) =
+                *reinterpret_cast<h4a*>(tk + 8192 + vw + ((f ^ (vc >> 2)) & 3) * 64) =
                     h4a{p01.x, p01.y, p23.x, p23.y};
             }
         }
@@ -1802,8 +1783,9 @@ int launch_attn_prefill(const AttnPrefill& P, hipStream_t st) {
         // 64-row, with the append, us: 100 tokens 13.5 / 13.8, 256: 21.5 / 17.4, 512: 41.3 /
         // 23.9, 1500: 144 / 63; 16 tokens after 8000: 304 / 161); four key groups to a
         // workgroup while one round of them holds the grid (1500: two groups 65.5, four 63.0;
-        // 2048, 640 workgroups: 88.4 / 103). Error against float64, 1500 / 8000 keys:
-        // 3.7e-8 / 5.3e-7 before, 3.2e-8 / 2.9e-7.
+        // 2048, 640 workgroups: 88.4 / 103). Error (2-norm) against float64, 1500 queries, 16 after
+        // 8000: 16-row kernel 2.0e-7, 8.2e-7, here 1.6e-7, 5.4e-7; with channels of six times the
+        // others 2.3e-7, 8.1e-7 and 1.9e-7, 5.5e-7.
         if (P.pos0 + P.n >= 256) {
             const dim3 fg((unsigned)P.Hkv, (unsigned)ceil_div(P.n, kFlashRows / G));
             const bool four = (int64_t)fg.x * fg.y <= 512;

@@ -143,6 +143,7 @@ struct tenzo_engine_opaque {
 
     // batched prefill (tenzo_hip_engine_prefill): rows of up to pf_cap tokens
     int pf_cap = 0;
+    int pf_rows = 0;  // rows of the last pass
     float* pf_x = nullptr;
     float* pf_h1 = nullptr;
     float* pf_qkv = nullptr;
@@ -705,7 +706,7 @@ int prefill_buffers(tenzo_engine_t e, int n) {
     const int want = n <= kPrefillRowsSmall ? kPrefillRowsSmall : kPrefillRows;
     if (e->pf_cap >= want) return TENZO_SUCCESS;
     TZ_HIP(hipStreamSynchronize(e->st));
-    e->pf_cap = 0;
+    e->pf_cap = e->pf_rows = 0;
     void** bufs[] = {(void**)&e->pf_x,  (void**)&e->pf_h1,    (void**)&e->pf_qkv, (void**)&e->pf_attn,
                      (void**)&e->pf_gu, (void**)&e->pf_codes, (void**)&e->pf_aq,  (void**)&e->pf_tok};
     for (void** b : bufs) {
@@ -891,6 +892,7 @@ int run_prefill(tenzo_engine_t e, const int32_t* tokens, int n, bool exact) {
         // the copy of the tokens and the next pass's buffers are reused
         TZ_HIP(hipStreamSynchronize(e->st));
         e->seq_len += m;
+        e->pf_rows = m;
     }
     TZ_HIP(hipMemcpyAsync(e->x, e->pf_x + (int64_t)(m - 1) * e->H, (size_t)e->H * 4,
                           hipMemcpyDeviceToDevice, e->st));
@@ -1686,7 +1688,9 @@ TENZO_HIP_API int tenzo_hip_engine_get_buffer(tenzo_engine_t e, const char* name
                 {"attn_out", e->attn, e->qd},
                 {"h1", e->h1, e->H},
                 {"gate_up", e->gu, 2 * (int64_t)e->F},
-                {"logits", e->logits, e->V}};
+                {"logits", e->logits, e->V},
+                {"prefill_qkv", e->pf_qkv, (int64_t)e->pf_rows * (e->qd + 2 * e->kvd)},
+                {"prefill_attn", e->pf_attn, (int64_t)e->pf_rows * e->qd}};
     for (const B& b : bufs) {
         if (std::strcmp(b.n, name) == 0) {
             TZ_CHECK(n >= b.len, "engine_get_buffer: %s needs %lld floats", name,

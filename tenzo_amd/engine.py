@@ -289,6 +289,16 @@ class Engine:
                  "logits": c.vocab_size}
         return out[:sizes[name]].copy()
 
+    def prefill_rows(self, name: str, rows: int) -> np.ndarray:
+        """[rows][..] of the last layer in the last batched-prefill pass, which had that many
+        tokens: "prefill_qkv" (q | k | v before RoPE) or "prefill_attn"."""
+        c = self.cfg
+        width = c.num_q_heads * 128 + (2 * c.num_kv_heads * 128 if name == "prefill_qkv" else 0)
+        out = np.zeros((rows, width), np.float32)
+        self._check(self.L.tenzo_hip_engine_get_buffer(self.h, name.encode(), _ptr(out), out.size),
+                    f"get_buffer({name})")
+        return out
+
     LAYER_STATE = {"x": (0, np.float32), "h1": (1, np.float32), "attn_out": (2, np.float32),
                    "acc_qkv": (3, np.int32), "acc_o": (4, np.int32), "acc_gu": (5, np.int32),
                    "acc_down": (6, np.int32)}

@@ -412,5 +412,100 @@ def test_engine_prefill_streaming_64_rows(torch_dev, ctx, n, Hq, Hkv):
             assert np.sqrt((d.astype(np.float64) ** 2).mean(axis=(0, 2))).max() < 4.0
 
 
+def _one_layer(eng_mod, synth, Hq, Hkv, ctx, n, loud, seed):
+    """A one-layer engine and its model. loud: embeddings with a common part, which rows 5 and 69
+    of each query head sum up while its other rows take differences of four values; the keys
+    hold zeros there."""
+    cfg = synth.DecodeConfig(hidden=128 * Hq, n_q_heads=Hq, n_kv_heads=Hkv, n_layers=1, ffn=512,
+                             vocab=1024, max_seq=ctx + n + 8, theta=10000.0)
+    sm = synth.make_model(cfg, seed=seed, ctx=ctx)
+    if loud:
+        rng = np.random.default_rng(seed)
+        sm.embed[:] = np.clip(np.rint(60 + 18 * rng.standard_normal(sm.embed.shape)), -127, 127)
+        lw, H = sm.layers[0], cfg.hidden
+        lw.in_norm[:] = 1.0
+        wq = np.zeros((Hq * 128, H), np.int8)
+        for r in wq:
+            r[rng.choice(H, 4, replace=False)] = [1, 1, -1, -1]
+        wk = formats.tl1_unpack(lw.tl1["k"], Hkv * 128, H).copy()
+        for d in (5, 69):
+            wq[d::128], wk[d::128] = 1, 0
+        sm.kc[:, :, :, [5, 69]] = 0
+        lw.tl1["q"], lw.tl1["k"] = formats.tl1_pack(wq), formats.tl1_pack(wk)
+        lw.scale["q"] = np.float32(8.0)
+    e = eng_mod.Engine(cfg)
+    e.set_model(sm)
+    return cfg, e
+
+
+def _attention64(torch, cfg, qkv, kv, pos0, table):
+    """softmax(q k / sqrt(128)) v of the rows' rotated queries (fp32, as the append and decode
+    rotate them) over the cached rows in float64: (output, largest |score|)."""
+    n, Hq, Hkv = len(qkv), cfg.n_q_heads, cfg.n_kv_heads
+    q = qkv[:, :Hq * 128].reshape(n, Hq, 128)
+    cs, sn = (t[pos0:pos0 + n, None] for t in (table[:, :64], table[:, 64:]))
+    lo, hi = q[..., :64], q[..., 64:]
+    d = np.float64
+    q = np.concatenate([(lo.astype(d) * cs - (hi * sn).astype(d)).astype(np.float32),
+                        (lo.astype(d) * sn + (hi * cs).astype(d)).astype(np.float32)], -1)
+    q = torch.from_numpy(q.astype(d)).cuda()
+    k, v = (torch.from_numpy(c[0].astype(d) * s[0, :, :, None].astype(d)).cuda()
+            for c, s in ((kv[0], kv[2]), (kv[1], kv[3])))
+    late = torch.arange(k.shape[1], device="cuda")[None] > pos0 + torch.arange(n, device="cuda")[:, None]
+    out, top = torch.empty((n, Hq, 128), dtype=torch.float64, device="cuda"), 0.0
+    for h in range(Hq):
+        s = (q[:, h] @ k[h * Hkv // Hq].T / 128 ** 0.5).masked_fill(late, -float("inf"))
+        top = max(top, s[~late].abs().max().item())
+        out[:, h] = torch.softmax(s, -1) @ v[h * Hkv // Hq]
+    return out.reshape(n, -1).cpu().numpy(), top
+
+
+@pytest.mark.parametrize("ctx,n,Hq,Hkv", [(0, 700, 4, 1), (900, 60, 4, 4), (1500, 200, 8, 1),
+                                          (0, 2048, 20, 5), (100, 60, 4, 2)])
+@pytest.mark.parametrize("loud", [False, True])
+def test_engine_prefill_streaming_error(torch_dev, ctx, n, Hq, Hkv, loud):
+    """Streaming attention outputs of a pass against float64 (the 64-row kernel with four and two
+    key groups, and the 16-row kernel), for ordinary queries and for rows whose largest elements, a
+    few hundred times the others, meet zero keys. A query element's hi and lo parts hold 22 bits
+    of it, a score of at most 32 is wrong by at most 32 (2^-22 + 2^-21 for its sums), so a
+    weight by 2.3e-5 of itself; over hundreds of keys with independent signs that is below
+    2e-6 of the output's norm."""
+    from tenzo_amd import _lib, engine as eng_mod, synth
+    cfg, e = _one_layer(eng_mod, synth, Hq, Hkv, ctx, n, loud, 31 + n)
+    toks = np.random.default_rng(n).integers(0, cfg.vocab, n).astype(np.int32)
+    table = np.empty((cfg.max_seq, 128), np.float32)
+    _lib.load().tenzo_hip_rope_table(10000.0, 128, 0, cfg.max_seq, table.ctypes.data)
+    print(f"streaming error ctx={ctx} n={n} Hq={Hq} Hkv={Hkv} loud={loud}", flush=True)
+    with e:
+        e.prefill_batch(toks)
+        qkv, out = e.prefill_rows("prefill_qkv", n), e.prefill_rows("prefill_attn", n)
+        ref, top = _attention64(torch_dev, cfg, qkv, e.get_kv(ctx + n), ctx, table)
+    q = np.abs(qkv[:, :Hq * 128]).reshape(n, Hq, 128)
+    spread = q.max() / np.median(q[q > 0])
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    print(f"error {err:.2e}, largest score {top:.1f}, largest |q| over the median {spread:.0f}", flush=True)
+    assert top < 32 and (spread > 200) == loud
+    assert err < 2e-6
+
+
+@pytest.mark.parametrize("scale", [np.nan, np.inf])
+@pytest.mark.parametrize("ctx,n,Hq,Hkv", [(0, 40, 4, 1), (900, 30, 4, 2), (0, 2048, 20, 5)])
+def test_engine_prefill_streaming_queries_not_finite(torch_dev, ctx, n, Hq, Hkv, scale):
+    """Queries of NaN (or of infinities and NaN) over finite keys and values: NaN outputs, as the
+    exact form gives, from the 16-row and the 64-row kernel alike."""
+    from tenzo_amd import engine as eng_mod, synth
+    cfg, e = _one_layer(eng_mod, synth, Hq, Hkv, ctx, n, False, 7)
+    sm = synth.make_model(cfg, seed=7, ctx=ctx)
+    sm.layers[0].scale["q"] = np.float32(scale)
+    e.set_layer(0, sm.layers[0])
+    toks = np.random.default_rng(n).integers(0, cfg.vocab, n).astype(np.int32)
+    with e:
+        for exact in (True, False):
+            e.rewind(ctx)
+            e.prefill_batch(toks, exact=exact)
+            assert np.isfinite(e.prefill_rows("prefill_qkv", n)[:, Hq * 128:]).all()
+            assert np.isnan(e.prefill_rows("prefill_attn", n)).all(), exact
+
+
 def rel(a, b):
     return np.abs(np.asarray(a, np.float64) - b).max() / max(np.abs(b).max(), 1e-30)
