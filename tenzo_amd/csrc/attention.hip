@@ -1456,32 +1456,31 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
         mr = mn;
 #pragma unroll
         for (int j = 0; j < 16; ++j) d[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(d[j], c2, -mc));
-        if (masked) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (t0 + 8 * (j >> 2) + 4 * g + (j & 3) > prow) d[j] = 0.0f;
-        }
-        float ls = 0.0f;
-        h8a wh[2], wl[2];
+        f16a w;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const float4 f = *reinterpret_cast<const float4*>(&vsl[kg][8 * q + 4 * g]);
             const float fs[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                ls += d[4 * q + e];
-                d[4 * q + e] = __fmul_rn(d[4 * q + e], fs[e]);  // (fs: s_v 2^e)
-            }
+            for (int e = 0; e < 4; ++e) w[4 * q + e] = __fmul_rn(d[4 * q + e], fs[e]);  // (fs: s_v 2^e)
         }
+        if (masked) {  // (a later token's scale may be an infinity: its products too)
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (t0 + 8 * (j >> 2) + 4 * g + (j & 3) > prow) d[j] = w[j] = 0.0f;
+        }
+        float ls = 0.0f;
+        h8a wh[2], wl[2];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
+            ls += d[j];
             // (opaque: fused with the product, one of hi's two uses would round once
             // instead of twice, and lo would not be its remainder on a tie)
-            float w = d[j];
-            asm("" : "+v"(w));
-            const _Float16 hi = (_Float16)w;
+            float x = w[j];
+            asm("" : "+v"(x));
+            const _Float16 hi = (_Float16)x;
             wh[j >> 3][j & 7] = hi;
-            wl[j >> 3][j & 7] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, w);
+            wl[j >> 3][j & 7] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, x);
         }
         lr = __builtin_fmaf(lr, rs, ls);
         const float dn = vdn[kg];
@@ -1557,8 +1556,8 @@ __global__ void __launch_bounds__(128 * KG, 2) attn_prefill_flash_kernel(AttnArg
             const float f = half_bits_to_float(sr);
             if (tid < 32 * KG) ksl[tid >> 5][tid & 31] = __fmul_rn(f, kScaleFactor);
             else {
-                // the tile's power-of-two scale of W = p * s_v, from its largest s_v
-                float mx = row16_max(f);
+                // the tile's power-of-two scale of W = p * s_v, from its largest finite s_v
+                float mx = row16_max(f < __builtin_inff() ? f : 0.0f);
                 mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
                 const int sh = fp16_span_exp(mx);
                 vsl[(tid >> 5) - KG][tid & 31] = ldexpf(f, sh);

@@ -507,5 +507,38 @@ def test_engine_prefill_streaming_queries_not_finite(torch_dev, ctx, n, Hq, Hkv,
             assert np.isnan(e.prefill_rows("prefill_attn", n)).all(), exact
 
 
+@pytest.mark.parametrize("n,Hq,Hkv", [(700, 4, 1), (2048, 20, 5), (1100, 8, 8)])
+def test_engine_prefill_streaming_infinite_scale(torch_dev, n, Hq, Hkv):
+    """A few tokens' value scales overflow fp16: the rows before such a token, also those of its
+    workgroup and those that share a key tile with it, have their ordinary outputs (against float64
+    as above), and the rows from it on are not finite, as in the exact form."""
+    from tenzo_amd import _lib, engine as eng_mod, synth
+    cfg, e = _one_layer(eng_mod, synth, Hq, Hkv, 0, n, False, 9)
+    sm = synth.make_model(cfg, seed=9, ctx=0)
+    toks = np.random.default_rng(n).permutation(max(n, cfg.vocab))[:n].astype(np.int32) % cfg.vocab
+    table = np.empty((cfg.max_seq, 128), np.float32)
+    _lib.load().tenzo_hip_rope_table(10000.0, 128, 0, cfg.max_seq, table.ctypes.data)
+    with e:
+        e.prefill_batch(toks)
+        top = np.sort(e.get_kv(n)[3].reshape(-1))[-3]
+        sm.layers[0].scale["v"] *= np.float32(66000.0 / top)  # (65520 and more round to infinity)
+        e.set_layer(0, sm.layers[0])
+        for exact in (True, False):
+            e.reset()
+            e.prefill_batch(toks, exact=exact)
+            out = e.prefill_rows("prefill_attn", n).reshape(n, Hkv, -1)
+            kv = e.get_kv(n)
+            far = np.isinf(kv[3][0])  # [Hkv][token]
+            assert 2 < far.sum() < 32
+            first = [int(f.argmax()) if f.any() else n for f in far]
+            print(f"n={n} exact={exact} first infinite scales {first}", flush=True)
+            kv = kv[:3] + (np.where(np.isinf(kv[3]), 0, kv[3]),)
+            ref, _ = _attention64(torch_dev, cfg, e.prefill_rows("prefill_qkv", n), kv, 0, table)
+            for h, p in enumerate(first):
+                assert not np.isfinite(out[p:, h]).any()
+                r = ref.reshape(n, Hkv, -1)[:p, h]
+                assert np.linalg.norm(out[:p, h] - r) < 2e-6 * np.linalg.norm(r), (exact, h)
+
+
 def rel(a, b):
     return np.abs(np.asarray(a, np.float64) - b).max() / max(np.abs(b).max(), 1e-30)
