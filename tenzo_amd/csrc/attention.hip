@@ -1778,14 +1778,21 @@ int launch_attn_prefill(const AttnPrefill& P, hipStream_t st) {
     if (rc) return rc;
     if (!P.exact && (G == 1 || G == 2 || G == 4 || G == 8)) {
         a.pos_n = P.n;
-        // The 64-row kernel from a prefix of 256 keys on (20 / 5 heads, 16-row kernel against
-        // 64-row, with the append, us: 100 tokens 13.5 / 13.8, 256: 21.5 / 17.4, 512: 41.3 /
-        // 23.9, 1500: 144 / 63; 16 tokens after 8000: 304 / 161); four key groups to a
-        // workgroup while one round of them holds the grid (1500: two groups 65.5, four 63.0;
-        // 2048, 640 workgroups: 88.4 / 103). Error (2-norm) against float64, 1500 queries, 16 after
+        // The 64-row kernel lays each key tile out once for 64 rows, but is a longer chain of
+        // steps a tile: it is the faster one from 256 keys on where the 16-row kernel has 192
+        // workgroups and more, from 384 at 96, else from 512, with fewer than 16 rows a kv head
+        // from 768 (20 / 5 heads, 16-row kernel against 64-row, with the append, us: 256 tokens
+        // 22.5 / 19.3, 512: 41.4 / 25.7, 1500: 137 / 61.4; 128 after 256: 21.7 / 21.4; 16 after
+        // 240: 17.3 / 18.6, after 496: 24.2 / 23.7, after 8000: 291 / 167; one after 511: 21.1 /
+        // 22.9, after 767: 27.5 / 27.7; for 1 to 8 heads a kv head within 3% of the better one).
+        // Four key groups to a workgroup while one round of them holds the grid (1500: two
+        // groups 67.9, four 65.2; 2048, 640 workgroups: 82.9 / 98.0). Error (2-norm) against
+        // float64, 1500 queries, 16 after
         // 8000: 16-row kernel 2.0e-7, 8.2e-7, here 1.6e-7, 5.4e-7; with channels of six times the
         // others 2.3e-7, 8.1e-7 and 1.9e-7, 5.5e-7.
-        if (P.pos0 + P.n >= 256) {
+        const int64_t groups16 = ceil_div(P.n, 16 / G) * P.Hkv;
+        if (P.pos0 + P.n >=
+            (groups16 >= 192 ? 256 : groups16 >= 96 ? 384 : P.n * G >= 16 ? 512 : 768)) {
             const dim3 fg((unsigned)P.Hkv, (unsigned)ceil_div(P.n, kFlashRows / G));
             const bool four = (int64_t)fg.x * fg.y <= 512;
 #define FLASH_CASE(GG)                                                                        \

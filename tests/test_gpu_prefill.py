@@ -382,11 +382,13 @@ def test_engine_prefill_streaming_attention(torch_dev, ctx, n, G):
 
 @pytest.mark.parametrize("ctx,n,Hq,Hkv", [(200, 60, 4, 4), (0, 256, 4, 2), (250, 77, 4, 1),
                                           (255, 1, 4, 1), (0, 300, 8, 1), (0, 2100, 16, 4),
-                                          (31, 2200, 16, 16)])
+                                          (31, 2200, 16, 16), (455, 60, 4, 4), (256, 256, 4, 2),
+                                          (450, 77, 4, 1), (767, 1, 4, 1), (0, 600, 8, 1)])
 def test_engine_prefill_streaming_64_rows(torch_dev, ctx, n, Hq, Hkv):
-    """The 64-row streaming attention (prefixes of 256 keys and more; four key groups
-    to a workgroup, two for the last two prompts) against the exact form, for every
-    count of heads per kv head, ragged ends of rows and of key tiles, and rows whose
+    """The streaming attention at and around the prefixes from which the 64-row kernel takes
+    over (512 keys; 768 for fewer than 16 rows a kv head, as the row of (767, 1); 384 and 256 where
+    the rows are many, as in the two prompts of over 2000 tokens, which have two key groups to a
+    workgroup, the others four) against the exact form, for every count of heads per kv head, ragged ends of rows and of key tiles, and rows whose
     prefix ends inside the first tiles. Each token's second-layer K and V codes come
     from its own first-layer attention: rounded codes may flip on a tie (a flip moves a
     few of a row's codes by one), a row with a key too many or too few differs
