@@ -1052,14 +1052,15 @@ TENZO_HIP_API int tenzo_hip_bitlinear_tl1_f32(const float* x, const void* w_pack
     if (K % 4 == 0 && Kp <= 8192 && tl1_pick_splits(N / 64, KS, M) == 1) {
         const dim3 grid((unsigned)(N / 64), (unsigned)M), blk(256);
         const uint4* wp = (const uint4*)w_packed;
-        // Several rows to a workgroup once there is one for every other CU: us at 24 rows,
-        // tl1_gemv_f32_kernel | 4 rows, 2560 x 6912 16.3 | 9.2, 2560 x 2560 7.8 | 5.8; at 8 rows
-        // of 3840 x 2560 5.9 | 5.6, of 2560 x 2560 (320 one-row blocks) 5.4 | 5.6. 8 rows share
-        // the unpacked weights of many workgroups: 300 rows of 2560 x 6912 51 | 44, 48 rows of
+        // Several rows to a workgroup once one row a workgroup gives every CU more than two, for
+        // rows over 2560 a little earlier: us, tl1_gemv_f32_kernel | 4 rows, 24 rows of 2560 x 6912
+        // 16.3 | 9.2, of 2560 x 2560 7.8 | 5.8; 12 rows of 2560 x 1028 (480 one-row blocks) 4.5 |
+        // 4.8, of 2560 x 2052 5.7 | 5.9, 16 rows 6.7 | 5.9; 12 of 2560 x 4096 7.4 | 6.5. 8 rows share the
+        // unpacked weights of many workgroups: 300 rows of 2560 x 6912 51 | 44, 48 rows of
         // 3840 x 2560 8.7 | 9.1. Short rows quantize in no time: 2560 x 256, 24 rows 3.8 | 4.0,
         // 48 rows 5.5 | 4.4.
         const int64_t blocks = N / 64 * M;
-        if (M >= 4 && blocks >= (K < 1024 ? 1536 : 480)) {
+        if (M >= 4 && blocks >= (K < 1024 ? 1536 : K <= 2560 ? 513 : 480)) {
             if (blocks >= 4096)
                 launch_tl1_rows_f32<8>(wp, x, M, N, K, KS, rs, y, st);
             else

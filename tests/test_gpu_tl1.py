@@ -102,11 +102,11 @@ def test_tl1_gemv_f32_entry_bit_exact(torch_dev, N, K, M):
         np.testing.assert_array_equal(y[m], yo)
 
 
-@pytest.mark.parametrize("N,K,M", [(512, 1028, 61), (512, 2500, 64), (1024, 6912, 31),
-                                   (4096, 8192, 67), (4096, 100, 66), (64, 2052, 481)])
+@pytest.mark.parametrize("N,K,M", [(512, 1028, 65), (512, 2500, 65), (1024, 6912, 31),
+                                   (4096, 8192, 67), (4096, 100, 66), (64, 2052, 513)])
 def test_tl1_f32_rows_bit_exact(torch_dev, N, K, M):
-    """Rows enough for the kernel that takes 4 or 8 of them (N / 64 * M from 480 on; K < 1024 from
-    1536; 8 from 4096): row groups and groups of four super-chunks end partly filled, K is not a
+    """Rows enough for the kernel that takes 4 or 8 of them (N / 64 * M from 513 on; K > 2560 from
+    480, K < 1024 from 1536; 8 from 4096): row groups and groups of four super-chunks end partly filled, K is not a
     multiple of 64. Every row equals the one-row call's bit for bit, also with an infinity or a NaN,
     the first ones the oracle's."""
     from tenzo_amd import ops
