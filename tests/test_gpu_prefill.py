@@ -58,6 +58,7 @@ def test_batch_equals_per_token_gemv(torch_dev, N, K, M):
 
 
 @pytest.mark.parametrize("M,N,K", [
+    (33, 4194368, 130),                                    # N above 2^22: tl1_mfma_kernel
     (5, 64, 64), (31, 320, 130), (64, 320, 1030),          # 64 x 32 tiles, four K groups
     (600, 1088, 200), (97, 8256, 64), (545, 1920, 320),    # 128 x 32, two K groups
     (1999, 1088, 130), (1030, 2112, 70), (260, 13824, 64),  # 128 x 64
@@ -78,6 +79,7 @@ def test_batch_shapes_against_whole_sums(torch_dev, M, N, K):
     wp = ops.tl1_repack(packed, N, K)
     codes, q, _ = ops.rmsnorm_quant31(torch.randn((M, K), device="cuda", generator=g))
     yb, ab = ops.bitlinear_tl1_batch(codes, q, wp, 0.0173, N, K, want_acc=True)
+    del u, nib, packed
     acc = codes[:, :K].double() @ w.double().T
     assert torch.equal(ab.double(), acc)
     scale = ops.actq_inv_scale(q) * torch.tensor(0.0173, device="cuda")
