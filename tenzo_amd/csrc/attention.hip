@@ -1827,22 +1827,25 @@ int launch_attn_prefill(const AttnPrefill& P, hipStream_t st) {
         while (s1 < P.n && pick_chunk(P.pos0 + s1 + 1, P.Hkv, 1) == T) ++s1;
         const int mc = (int)ceil_div(P.pos0 + s1, T);  // chunks of the run's last query
         const size_t per_query = (size_t)P.Hq * mc * kPartStride * 4;
-        const int qg_max =
+        int qg_max =
             mc > 1 ? (int)std::max<size_t>(1, std::min<size_t>(s1 - s0, (256u << 20) / per_query))
                    : s1 - s0;
-        for (int i0 = s0; i0 < s1; i0 += qg_max) {
-            const int n = std::min(qg_max, s1 - i0);
+        for (int i0 = s0, n; i0 < s1; i0 += n) {
+            n = std::min(qg_max, s1 - i0);
             a.pos = P.pos0 + i0;
-            a.pos_n = n;
             a.T = T;
             a.q = P.q + (int64_t)i0 * P.row_stride;
             a.out = P.out + (int64_t)i0 * P.out_stride;
             a.max_chunks = mc;
             a.part = nullptr;
-            if (mc > 1) {
+            while (mc > 1 && !a.part) {  // (fewer queries at a time where memory does not hold all)
                 a.part = (float*)Scratch::get(kScratchAttn, (size_t)n * per_query, st);
-                if (!a.part) return TENZO_ERROR_OUT_OF_MEMORY;
+                if (a.part) break;
+                if (n == 1) return TENZO_ERROR_OUT_OF_MEMORY;
+                (void)hipGetLastError();  // (the next launch's check would report it)
+                n = qg_max = (n + 1) / 2;
             }
+            a.pos_n = n;
             const dim3 grid((unsigned)mc, (unsigned)P.Hkv, (unsigned)ceil_div(n, QB));
             const int U = T / 32;  // 2 .. 8 (pick_chunk: multiples of 32 from 64 to kMaxChunk)
             if (U == 2) {  // 64-token chunks: the kernel with the score tile sized to them

@@ -144,6 +144,7 @@ struct tenzo_engine_opaque {
     // batched prefill (tenzo_hip_engine_prefill): rows of up to pf_cap tokens
     int pf_cap = 0;
     int pf_rows = 0;  // rows of the last pass
+    int pf_most = 0;  // rows of a pass that memory held, once it did not hold the wanted ones
     float* pf_x = nullptr;
     float* pf_h1 = nullptr;
     float* pf_qkv = nullptr;
@@ -698,17 +699,14 @@ int load_model_files(tenzo_engine_t e, const char* weights_path, const char* mli
 // rows fill the chip with 256 x 128 tiles of every projection (1500 tokens through four
 // layers and a decode step: 2.23 ms in three passes of 512 rows and with the activation
 // left to the quantizer, 1.61 ms in one pass with it in the gate | up product). The
-// buffers hold kPrefillRowsSmall rows for prompts up to that length, else a whole pass.
+// buffers hold the prompt's rows in steps of kPrefillStep, as many as there is memory for.
 constexpr int kPrefillRows = 2048;
-constexpr int kPrefillRowsSmall = 512;
+constexpr int kPrefillStep = 512;
 
-int prefill_buffers(tenzo_engine_t e, int n) {
-    const int want = n <= kPrefillRowsSmall ? kPrefillRowsSmall : kPrefillRows;
-    if (e->pf_cap >= want) return TENZO_SUCCESS;
-    TZ_HIP(hipStreamSynchronize(e->st));
-    e->pf_cap = e->pf_rows = 0;
+int prefill_free(tenzo_engine_t e) {
     void** bufs[] = {(void**)&e->pf_x,  (void**)&e->pf_h1,    (void**)&e->pf_qkv, (void**)&e->pf_attn,
                      (void**)&e->pf_gu, (void**)&e->pf_codes, (void**)&e->pf_aq,  (void**)&e->pf_tok};
+    e->pf_cap = e->pf_rows = 0;
     for (void** b : bufs) {
         void* p = *b;
         if (!p) continue;
@@ -716,18 +714,34 @@ int prefill_buffers(tenzo_engine_t e, int n) {
         e->allocs.erase(std::find(e->allocs.begin(), e->allocs.end(), p));
         TZ_HIP(hipFree(p));
     }
-    const size_t R = want;
-    const int64_t Kp = std::max(ceil_div(e->F, 64), ceil_div(e->H, 64)) * 64;
-    int rc;
-    if ((rc = alloc_t(e, &e->pf_x, R * e->H * 4)) || (rc = alloc_t(e, &e->pf_h1, R * e->H * 4)) ||
-        (rc = alloc_t(e, &e->pf_qkv, R * (e->qd + 2 * e->kvd) * 4)) ||
-        (rc = alloc_t(e, &e->pf_attn, R * e->qd * 4)) ||
-        (rc = alloc_t(e, &e->pf_gu, R * 2 * e->F * 4)) ||
-        (rc = alloc_t(e, &e->pf_codes, R * Kp, true)) ||
-        (rc = alloc_t(e, &e->pf_aq, R * sizeof(tenzo_hip_actq_t))) ||
-        (rc = alloc_t(e, &e->pf_tok, R * 4)))
-        return rc;
-    e->pf_cap = want;
+    return TENZO_SUCCESS;
+}
+
+int prefill_buffers(tenzo_engine_t e, int n) {
+    const int most = e->pf_most ? e->pf_most : kPrefillRows;
+    for (int want = std::min((int)ceil_div(n, kPrefillStep) * kPrefillStep, most); e->pf_cap < want;
+         want -= kPrefillStep) {
+        TZ_HIP(hipStreamSynchronize(e->st));
+        int rc = prefill_free(e);
+        if (rc) return rc;
+        const size_t R = want;
+        const int64_t Kp = std::max(ceil_div(e->F, 64), ceil_div(e->H, 64)) * 64;
+        const size_t gu = tl1_mfma_glu_fits(want, e->F, e->H) ? e->F : 2 * (size_t)e->F;
+        if (!((rc = alloc_t(e, &e->pf_x, R * e->H * 4)) || (rc = alloc_t(e, &e->pf_h1, R * e->H * 4)) ||
+              (rc = alloc_t(e, &e->pf_qkv, R * (e->qd + 2 * e->kvd) * 4)) ||
+              (rc = alloc_t(e, &e->pf_attn, R * e->qd * 4)) ||
+              (rc = alloc_t(e, &e->pf_gu, R * gu * 4)) ||
+              (rc = alloc_t(e, &e->pf_codes, R * Kp, true)) ||
+              (rc = alloc_t(e, &e->pf_aq, R * sizeof(tenzo_hip_actq_t))) ||
+              (rc = alloc_t(e, &e->pf_tok, R * 4)))) {
+            e->pf_cap = want;
+            break;
+        }
+        (void)prefill_free(e);
+        if (rc != TENZO_ERROR_OUT_OF_MEMORY || want <= kPrefillStep) return rc;
+        (void)hipGetLastError();  // (the next launch's check would report it)
+        e->pf_most = want - kPrefillStep;
+    }
     return TENZO_SUCCESS;
 }
 

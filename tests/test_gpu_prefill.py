@@ -416,6 +416,42 @@ def test_engine_prefill_streaming_64_rows(torch_dev, ctx, n, Hq, Hkv):
             assert np.sqrt((d.astype(np.float64) ** 2).mean(axis=(0, 2))).max() < 4.0
 
 
+def test_engine_prefill_little_memory(torch_dev):
+    """A prompt of 2200 tokens where memory holds the buffers of one step of 512 rows only, and
+    scratch for a part of the queries: passes of as many rows as fit, bit for bit the same state,
+    and a longer prompt later takes no more either."""
+    from tenzo_amd import engine as eng_mod, synth
+    torch = torch_dev
+    cfg = synth.DecodeConfig(hidden=512, n_q_heads=4, n_kv_heads=1, n_layers=1, ffn=32768,
+                             vocab=512, max_seq=2304, theta=10000.0)
+    sm = synth.make_model(cfg, seed=3, ctx=0)
+    toks = np.random.default_rng(3).integers(0, cfg.vocab, 2200).astype(np.int32)
+    a, b = _engine_pair(eng_mod, cfg, sm)
+    hold = []
+    with a, b:
+        a.prefill_batch(toks, exact=True)  # 340 MiB for 2048 rows (512: 85), scratch up to 142
+        eng_mod.lib().tenzo_hip_release_scratch()
+        torch.cuda.empty_cache()
+        try:
+            for _ in range(8):
+                torch.cuda.synchronize()
+                free = torch.cuda.mem_get_info()[0]
+                if free < 122 << 20:
+                    break
+                hold.append(torch.empty(free - (112 << 20), dtype=torch.uint8, device="cuda"))
+            print("little memory: bytes left", free, flush=True)
+            assert free < 122 << 20
+            b.prefill_batch(toks[:600], exact=True)
+            b.prefill_batch(toks[600:], exact=True)
+        finally:
+            hold.clear()
+            torch.cuda.empty_cache()
+            eng_mod.lib().tenzo_hip_release_scratch()
+        for x, y in zip(a.get_kv(2200), b.get_kv(2200)):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_array_equal(a.buffer("x"), b.buffer("x"))
+
+
 def _one_layer(eng_mod, synth, Hq, Hkv, ctx, n, loud, seed):
     """A one-layer engine and its model. loud: embeddings with a common part, which rows 5 and 69
     of each query head sum up while its other rows take differences of four values; the keys
