@@ -545,10 +545,10 @@ q4_0_f16_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w,
 //
 // y[b][n] = sum over blocks of d_n * sum_j a_bj q_nj. An activation enters as the sum of
 // bf16 parts, each the truncation of what the ones before leave: three hold every bit of an
-// fp32 number, two those of an fp16 number, whatever its neighbours' magnitudes (a number
-// common to the block would take bits from small elements beside a large one). The codes are
-// exact in bf16 (a Q4_0 nibble as (q - 8) / 16), so all products are exact; two
-// v_mfma_f32_32x32x16_bf16 a block multiply the parts (first operand, row 8 j + b: part j of
+// fp32 number (but bits below 2^-133), two those of an fp16 number, whatever its neighbours'
+// magnitudes (a scale common to the block would take bits from small elements beside a large
+// one). The codes are exact in bf16 (a Q4_0 nibble as (q - 8) / 16), so all products are exact;
+// two v_mfma_f32_32x32x16_bf16 a block multiply the parts (first operand, row 8 j + b: part j of
 // activation row b) by 32 weight rows' codes (second operand). Lane l = 32 g + n then holds
 // weight row n's sums for activation rows 4 g + e (e < 4) in registers 4 j + e, and adds d_n
 // (the parts' sums, smallest first) to its fp32 sums. MFMA step s takes elements 16 g + 8 s ..
