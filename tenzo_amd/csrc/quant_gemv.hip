@@ -558,15 +558,15 @@ q4_0_f16_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w,
 //
 // A workgroup owns 32 weight rows; wave v takes blocks 8 v .. 8 v + 7 of each chunk of 8 W
 // blocks by itself (its activations and weights go through LDS of its own, no barriers), and
-// the waves' sums are added in LDS pairwise at the end. Neighbouring lanes fetch neighbouring
+// the waves' sums are added in LDS at the end, with what those sums and the chunks' round off. Neighbouring lanes fetch neighbouring
 // 16 bytes of a row's 8 blocks (lanes that read whole blocks, or their own MFMA row, cost the
 // address unit a clock each: 1.5 and 3 times the time), one chunk ahead, and leave them in
 // LDS as they are. What is left is vector work: splitting the activations (the same ones in
 // every workgroup) and converting the codes.
-// 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 17.9 | 39.2, 16 rows 27.0 | 101
-// (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 15.9 | 26.9. Error against 64 bits
-// (2-norm) of 11008 x 11008: fp32 rows 8.7e-8 | 1.3e-7, fp16 rows 8.3e-8 | 8.5e-8 (Q4_0), 8.6e-8 |
-// 8.9e-8 (Q8_0); 9.1e-8 and 9.2e-8 if a wave's chunks are one chain of sums.
+// 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 18.4 | 41.2, 16 rows 28.0 | 99.7
+// (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 16.2 | 27.7. Error against 64 bits
+// (2-norm) of 5504 x 14336: fp32 rows 6.2e-8 | 1.3e-7, fp16 rows 5.7e-8 | 8.6e-8 (Q4_0), 6.1e-8 |
+// 9.1e-8 (Q8_0); with plain sums of the chunks and waves (1% faster) 8.7e-8 and more.
 // ------------------------------------------------------------------------
 typedef __bf16 gb8 __attribute__((ext_vector_type(8)));
 typedef float gf16 __attribute__((ext_vector_type(16)));
@@ -602,6 +602,13 @@ __device__ __forceinline__ void wave_lds_order() {
 // two fp32 numbers' high halves (exact where the low halves are zero)
 __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+// s += v; low collects what the additions round off (exactly: Knuth's two-sum)
+__device__ __forceinline__ void add_exact(float& s, float& low, float v) {
+    const float t = s + v, u = t - s;
+    low += (s - (t - u)) + (v - u);
+    s = t;
 }
 
 template <bool Q4, typename TA, int W>  // W waves
@@ -740,8 +747,7 @@ gguf_rows_kernel(const TA* __restrict__ act, const uint8_t* __restrict__ w, floa
         return Q4 ? 16.0f * d : d;
     };
 
-    float acc[4] = {}, run[4] = {};  // activation rows 4 g + e; the last 1 to 4 chunks apart
-    int nrun = 0;
+    float acc[4] = {}, low[4] = {};  // activation rows 4 g + e: the chunks' sum, what it rounded off
     load_acts(8 * wave, x[0]);
     load_acts(8 * wave + 4, x[1]);
     load_codes(8 * wave);
@@ -771,29 +777,27 @@ gguf_rows_kernel(const TA* __restrict__ act, const uint8_t* __restrict__ w, floa
             wave_lds_order();
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) run[e] += sum[e];
-        if (++nrun == 4) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += run[e], run[e] = 0.0f;
-            nrun = 0;
-        }
+        for (int e = 0; e < 4; ++e) add_exact(acc[e], low[e], sum[e]);
     }
     __syncthreads();
-    float* red = reinterpret_cast<float*>(part);  // [wave][activation row][weight row]
+    float2* red = reinterpret_cast<float2*>(part);  // [wave][activation row][weight row]
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[(wave * 8 + 4 * g + e) * 32 + n] = acc[e] + run[e];
+    for (int e = 0; e < 4; ++e) red[(wave * 8 + 4 * g + e) * 32 + n] = make_float2(acc[e], low[e]);
     __syncthreads();
     if (tid < 256) {
         const int b = tid >> 5;
         if (row0 + n < N && b < nb) {
-            float v[W];
+            float2 v[W];
 #pragma unroll
             for (int q = 0; q < W; ++q) v[q] = red[(q * 8 + b) * 32 + n];
+            float sum = v[0].x, rest = v[0].y;
 #pragma unroll
-            for (int h = W / 2; h; h >>= 1)
-#pragma unroll
-                for (int q = 0; q < h; ++q) v[q] += v[q + h];
-            y[(int64_t)(b0 + b) * N + row0 + n] = v[0];
+            for (int q = 1; q < W; ++q) {
+                rest += v[q].y;
+                add_exact(sum, rest, v[q].x);
+            }
+            // (a sum that is not finite leaves NaN)
+            y[(int64_t)(b0 + b) * N + row0 + n] = rest == rest ? sum + rest : sum;
         }
     }
 }
