@@ -558,11 +558,11 @@ q4_0_f16_kernel(const uint16_t* __restrict__ act, const uint8_t* __restrict__ w,
 //
 // A workgroup owns 32 weight rows; wave v takes blocks 8 v .. 8 v + 7 of each chunk of 8 W
 // blocks by itself (its activations and weights go through LDS of its own, no barriers), and
-// the waves' sums are added in LDS at the end, with what those sums and the chunks' round off. Neighbouring lanes fetch neighbouring
-// 16 bytes of a row's 8 blocks (lanes that read whole blocks, or their own MFMA row, cost the
-// address unit a clock each: 1.5 and 3 times the time), one chunk ahead, and leave them in
-// LDS as they are. What is left is vector work: splitting the activations (the same ones in
-// every workgroup) and converting the codes.
+// the waves' sums are added in LDS at the end, with what those sums and the chunks' round off.
+// Neighbouring lanes fetch neighbouring 16 bytes of a row's 8 blocks (lanes that read whole
+// blocks, or their own MFMA row, cost the address unit a clock each: 1.5 and 3 times the time),
+// one chunk ahead, and leave them in LDS as they are. What is left is vector work: splitting the
+// activations (the same ones in every workgroup) and converting the codes.
 // 11008 x 4096, us, here | the kernels above: Q8_0 fp32 6 rows 18.4 | 41.2, 16 rows 28.0 | 99.7
 // (49 MB of weights: 10 us at 5 TB/s); Q4_0 fp16 8 rows 16.2 | 27.7. Error against 64 bits
 // (2-norm) of 5504 x 14336: fp32 rows 6.2e-8 | 1.3e-7, fp16 rows 5.7e-8 | 8.6e-8 (Q4_0), 6.1e-8 |
