@@ -1709,6 +1709,7 @@ TENZO_HIP_API int tenzo_hip_engine_get_buffer(tenzo_engine_t e, const char* name
         if (std::strcmp(b.n, name) == 0) {
             TZ_CHECK(n >= b.len, "engine_get_buffer: %s needs %lld floats", name,
                      (long long)b.len);
+            if (b.len == 0) return TENZO_SUCCESS;
             TZ_HIP(hipSetDevice(e->dev));
             TZ_HIP(hipStreamSynchronize(e->st));
             TZ_HIP(hipMemcpy(out, b.p, (size_t)b.len * 4, hipMemcpyDeviceToHost));

@@ -218,7 +218,7 @@ def test_engine_prefill_passes(torch_dev):
 
 
 def test_engine_prefill_longer_than_one_pass(torch_dev):
-    """600 tokens: more than the small buffers' 512 rows, attention over up to 19
+    """600 tokens: more than one step of 512 buffer rows, attention over up to 19
     chunks per query, G = 4 query heads per kv head."""
     from tenzo_amd import engine as eng_mod, synth
     cfg = synth.DecodeConfig(hidden=512, n_q_heads=4, n_kv_heads=1, n_layers=2, ffn=512,
@@ -320,6 +320,7 @@ def test_engine_prefill_errors(torch_dev):
         with pytest.raises(RuntimeError, match="full"):
             e.prefill_batch(np.zeros(17, np.int32))
         assert e.seq_len == 0
+        assert not e.prefill_rows("prefill_attn", 3).any()  # (no pass yet: nothing is copied)
         e.prefill_batch(np.zeros(16, np.int32))
         assert e.seq_len == 16
 

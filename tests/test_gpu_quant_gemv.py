@@ -193,6 +193,32 @@ def test_gguf_rows_wide_blocks(torch_dev, kind, N, K, B):
         assert ((y - ref).norm() / ref.norm()).item() < 2.7e-7, factor
 
 
+@pytest.mark.parametrize("offset", [2, 4, 8])
+@pytest.mark.parametrize("kind", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("f16a", [False, True])
+def test_gguf_rows_weight_alignment(torch_dev, kind, offset, f16a):
+    """Weights at 4 and 8 bytes past a 16-byte line go to the matrix-core kernel, at 2 bytes to the
+    others: the sums of the aligned weights up to fp32 rounding (about 20 of 2^-24, both sides)."""
+    from tenzo_amd import ops
+    torch = torch_dev
+    N, K, B = 4100, 1024, 9
+    rng = np.random.default_rng(offset)
+    d = (0.002 + 0.004 * rng.random((N, K // 32))).astype(np.float16)
+    if kind == "q4_0":
+        w = formats.q4_0_pack(rng.integers(0, 16, size=(N, K), dtype=np.uint8), d)
+    else:
+        w = formats.q8_0_pack(rng.integers(-128, 128, size=(N, K)).astype(np.int8), d)
+    w = dev(torch, np.asarray(w).view(np.uint8).reshape(-1))
+    moved = torch.empty(w.numel() + 16, dtype=torch.uint8, device="cuda")[offset:offset + w.numel()]
+    moved.copy_(w)
+    assert moved.data_ptr() % 16 == offset
+    a = dev(torch, rng.standard_normal((B, K)).astype(np.float32))
+    a = a.half() if f16a else a
+    run = getattr(ops, "gemv_" + kind)
+    y, z = run(a, w, K, N).double(), run(a, moved, K, N).double()
+    assert ((y - z).norm() / y.norm()).item() < 4e-7
+
+
 @pytest.mark.parametrize("N,K", [(64, 32), (11008, 4096), (100, 2304), (257, 8192), (33, 288)])
 def test_q4_0_q8_0_activations(torch_dev, N, K):
     from tenzo_amd import ops
