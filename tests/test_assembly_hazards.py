@@ -59,7 +59,7 @@ def hazards(lines):
     return bad
 
 
-def test_checker_sees_a_planted_hazard():
+def test_a_planted_hazard_is_seen():
     load = ("buffer_load_dwordx4 v1, s[12:15], 0 offen lds", True)
     late = [("v_readlane_b32 s13, v40, 3", False), ("s_mov_b32 m0, s4", True), ("s_nop 0", True), load]
     assert hazards(late) and not hazards(late[:1] + [("s_nop 4", False)] + late[1:])
